@@ -93,6 +93,27 @@ int stm_nf4_dequantize_many(int count, const uint8_t* const* packed, const float
                             int blocksize, void* const* out, int out_dtype, void* stream);
 
 /*
+ * stm_nf4_dequantize_many for payloads in pinned host memory: packed[t] and
+ * absmax[t] are host addresses (hipHostMalloc) that the kernel reads over the
+ * host link, so the payload crosses it once and needs no device copy
+ * (the two uploads and the dequantize per parameter of stratum/upload.py
+ * ensure_weights, :1022-1044). Same results, bit for bit. The caller keeps the
+ * memory allocated until the launch has run. STM_ERR_UNSUPPORTED, before any
+ * launch, for more than 32 tensors, n[t] % 8 != 0, unaligned pointers (4 bytes
+ * in, 16 out) and memory that is not one pinned host range.
+ */
+int stm_nf4_dequantize_host(int count, const uint8_t* const* packed, const float* const* absmax, const int64_t* n,
+                            int blocksize, void* const* out, int out_dtype, void* stream);
+
+/*
+ * 1 if the work recorded before a HIP event is done, 0 if not, negative on an
+ * error; allowed while another thread captures a graph. No counterpart in the
+ * reference: the caller of stm_nf4_dequantize_host learns with it when the
+ * payload may be freed.
+ */
+int stm_event_done(void* event);
+
+/*
  * Fused NF4 dequant-GEMM, forward of a frozen Linear:
  *   Y[M, N] = X[M, K] . W[N, K]^T  (+ bias[N])  (+ T[M, R] . L[N, R]^T)
  * with W given as NF4 (packed [N*K/2], absmax [N*K/blocksize]) and dequantized

@@ -243,6 +243,38 @@ int stm_nf4_dequantize_many(int count, const uint8_t* const* packed, const float
     return launch_dequantize_many(count, packed, absmax, n, blocksize, out, out_dtype, (hipStream_t)stream);
 }
 
+int stm_nf4_dequantize_host(int count, const uint8_t* const* packed, const float* const* absmax, const int64_t* n,
+                            int blocksize, void* const* out, int out_dtype, void* stream) {
+    g_err[0] = 0;
+    if (count < 0) return set_error(STM_ERR_INVALID, "dequantize_host: count %d < 0", count);
+    if (!valid_dtype(out_dtype)) return set_error(STM_ERR_INVALID, "dequantize_host: bad dtype %d", out_dtype);
+    if (!valid_blocksize(blocksize))
+        return set_error(STM_ERR_INVALID, "dequantize_host: blocksize %d not a power of two in [64, 4096]", blocksize);
+    if (count == 0) return STM_OK;
+    if (!packed || !absmax || !n || !out) return set_error(STM_ERR_INVALID, "dequantize_host: NULL array");
+    for (int t = 0; t < count; ++t) {
+        if (n[t] < 0) return set_error(STM_ERR_INVALID, "dequantize_host: n[%d] = %lld < 0", t, (long long)n[t]);
+        if (n[t] > 0 && (!packed[t] || !absmax[t] || !out[t]))
+            return set_error(STM_ERR_INVALID, "dequantize_host: NULL pointer for tensor %d", t);
+    }
+    return launch_dequantize_host(count, packed, absmax, n, blocksize, out, out_dtype, (hipStream_t)stream);
+}
+
+int stm_event_done(void* event) {
+    g_err[0] = 0;
+    if (!event) return set_error(STM_ERR_INVALID, "event_done: NULL event");
+    // a query is not part of what another thread may be capturing
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    hipError_t e = hipThreadExchangeStreamCaptureMode(&mode);
+    if (e != hipSuccess) return set_error(STM_ERR_HIP, "event_done: %s", hipGetErrorString(e));
+    e = hipEventQuery((hipEvent_t)event);
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    if (e == hipSuccess) return 1;
+    (void)hipGetLastError();  // hipErrorNotReady is not an error of a later launch
+    if (e == hipErrorNotReady) return 0;
+    return set_error(STM_ERR_HIP, "event_done: %s", hipGetErrorString(e));
+}
+
 static int check_gemm_common(const char* who, const void* a, const uint8_t* packed, const float* absmax,
                              const void* out, int64_t M, int64_t N, int64_t K, int blocksize, int dtype) {
     if (!is_16bit(dtype)) return set_error(STM_ERR_INVALID, "%s: dtype %d is not bf16/fp16", who, dtype);

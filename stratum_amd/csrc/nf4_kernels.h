@@ -69,6 +69,9 @@ int launch_quantize_many(int count, const void* const* A, const int64_t* n, int 
                          uint8_t* const* packed, float* const* absmax, hipStream_t stream);
 int launch_dequantize_many(int count, const uint8_t* const* packed, const float* const* absmax, const int64_t* n,
                            int bs, void* const* out, int out_dtype, hipStream_t stream);
+// Payloads in pinned host memory, read by the kernel over the host link.
+int launch_dequantize_host(int count, const uint8_t* const* packed, const float* const* absmax, const int64_t* n,
+                           int bs, void* const* out, int out_dtype, hipStream_t stream);
 int launch_gemm_fwd(const GemmArgs& g, int dtype, hipStream_t stream);
 int launch_gemm_bwd(const GemmArgs& g, int dtype, hipStream_t stream);
 

@@ -322,6 +322,41 @@ def dequantize_4bit_many(items: Sequence[tuple], *, dtype: Optional[torch.dtype]
 
 
 @torch.no_grad()
+def dequantize_4bit_host(items: Sequence[tuple], device: torch.device) -> Optional[list]:
+    """:func:`dequantize_4bit_many` for payloads in pinned host memory: the kernel
+    reads the packed codes and absmax over the host link, so nothing is copied to
+    *device* first. None where that does not apply (more than 32 tensors, pageable
+    or unaligned memory, ...). The caller keeps the payloads until the current
+    stream has run the launch."""
+    import ctypes
+    states = [st for _, st in items]
+    if len({(st.blocksize, st.dtype) for st in states}) != 1:
+        return None
+    blocksize, dtype = states[0].blocksize, states[0].dtype
+    _check_nf4("nf4", blocksize)
+    ns = []
+    for q, st in items:
+        n = 1
+        for d in st.shape:
+            n *= int(d)
+        if (st.quant_type != "nf4" or q.is_cuda or st.absmax.is_cuda or q.dtype != torch.uint8
+                or st.absmax.dtype != torch.float32 or not q.is_contiguous() or not st.absmax.is_contiguous()
+                or q.numel() * 2 < n or st.absmax.numel() < -(-n // blocksize)):
+            return None
+        ns.append(n)
+    outs = [torch.empty(tuple(st.shape), dtype=dtype, device=device) for st in states]
+    with torch.cuda.device(device):
+        rc = _lib.lib().stm_nf4_dequantize_host(
+            len(items), _ptr_array([q.data_ptr() for q, _ in items]),
+            _ptr_array([st.absmax.data_ptr() for st in states]), _ptr_array(ns, ctypes.c_int64), blocksize,
+            _ptr_array([o.data_ptr() for o in outs]), _lib.dtype_tag(dtype), _lib.stream_handle(device))
+    if rc == _lib.STM_ERR_UNSUPPORTED:
+        return None
+    _lib.check(rc, "stm_nf4_dequantize_host")
+    return outs
+
+
+@torch.no_grad()
 def stack_nf4(items: Sequence[tuple]) -> tuple:
     """One NF4 weight ``[sum N_i, K]`` from weights ``[N_i, K]`` that share K and
     the blocksize: ``(packed, QuantState)`` with the packed bytes and absmax of

@@ -19,8 +19,9 @@ How this implementation is organised:
   ``free_weights`` / ``prefetch_weights`` therefore do not walk
   ``named_modules`` on every call.
 * **One materialisation routine** (``_materialise``) for the three staged
-  kinds: an NF4 payload is copied host-to-device (pinned memory, asynchronous)
-  and dequantized by the GPU kernel; an FP16-staged payload is copied; a plain
+  kinds: an NF4 payload is dequantized by the GPU kernel, which reads it where
+  it lies in pinned memory (a prefetched one from its device copy); an
+  FP16-staged payload is copied; a plain
   frozen parameter on the wrong device is moved. ``ensure_weights``,
   ``NF4Prefetch.finalize`` and ``upload_stream`` all go through it.
 * **Consumer streams.** A tensor materialised on a side stream is read by
@@ -39,6 +40,7 @@ from __future__ import annotations
 
 import hashlib
 import re
+import threading
 import time
 import weakref
 from dataclasses import dataclass
@@ -47,7 +49,9 @@ from typing import Iterable, Iterator, Optional, Sequence
 
 import torch
 
-from .functional import DEFAULT_ROUNDING, QuantState, dequantize_4bit_many, get_4bit_type, quantize_4bit
+from . import _lib
+from .functional import (DEFAULT_ROUNDING, QuantState, dequantize_4bit_host, dequantize_4bit_many, get_4bit_type,
+                         quantize_4bit)
 from .utils import log_event
 
 NF4_ATTR = "roundpipe_nf4_payload"
@@ -471,25 +475,65 @@ def _upload_nf4(payload: NF4Payload, device: torch.device):
     return (payload.quantized.to(device, non_blocking=True), payload.absmax.to(device, non_blocking=True))
 
 
+# Payloads that a launch still reads from pinned memory, with the event behind
+# it: a payload that its owner drops meanwhile must not be reused by the host.
+_host_reads: list = []
+_host_reads_lock = threading.Lock()
+
+
+def _keep_while_read(payloads: list, device: torch.device) -> None:
+    if torch.cuda.is_current_stream_capturing():
+        return  # what a graph reads is its owner's to keep, as with a captured copy
+    done = torch.cuda.Event()
+    done.record(torch.cuda.current_stream(device))
+    with _host_reads_lock:
+        _host_reads.append((done, payloads))
+
+
+def _release_host_reads() -> None:
+    if not _host_reads:
+        return
+    with _host_reads_lock:
+        _host_reads[:] = [r for r in _host_reads if _lib.lib().stm_event_done(r[0].cuda_event) == 0]
+
+
 def _materialise_nf4(entries: list, device: torch.device, consumers: list) -> int:
-    """Bring NF4 parameters to *device* on the current stream: H2D of each packed
-    payload (or its prefetched copy), then one batched dequantize per
-    (blocksize, dtype) group -- a layer's projections in one launch.
+    """Bring NF4 parameters to *device* on the current stream, one launch per
+    (blocksize, dtype) group, a layer's projections together. Payloads in pinned
+    memory are read by that launch where they lie; others (and prefetched ones,
+    which are there already) are dequantized from their device copy.
     *entries*: (slot, param, payload, prefetched (q, absmax) or None)."""
     if not entries:
         return 0
     groups: dict = {}
+    for entry in entries:
+        payload = entry[2]
+        groups.setdefault((payload.blocksize, payload.dtype, entry[3] is None), []).append(entry)
+    _release_host_reads()
     with torch.cuda.device(device):
-        for slot, p, payload, prefetched in entries:
-            q_dev, a_dev = prefetched if prefetched is not None else _upload_nf4(payload, device)
-            state = QuantState(absmax=a_dev, shape=payload.shape, code=payload.code, blocksize=payload.blocksize,
-                               quant_type=payload.quant_type, dtype=payload.dtype)
-            groups.setdefault((payload.blocksize, payload.dtype), []).append((slot, p, q_dev, state))
-        for members in groups.values():
-            weights = dequantize_4bit_many([(q, st) for _, _, q, st in members])
-            for (slot, p, _, _), w in zip(members, weights):
-                _replace_param_data(p, _hand_over(w, consumers), owner=slot.owner, pname=slot.name)
+        for (_, _, on_host), members in groups.items():
+            for at in range(0, len(members), 32):
+                _materialise_group(members[at:at + 32], device, consumers, on_host)
     return len(entries)
+
+
+def _materialise_group(members: list, device: torch.device, consumers: list, on_host: bool) -> None:
+    def items(sources):
+        return [(q, QuantState(absmax=a, shape=payload.shape, code=payload.code, blocksize=payload.blocksize,
+                               quant_type=payload.quant_type, dtype=payload.dtype))
+                for (_, _, payload, _), (q, a) in zip(members, sources)]
+
+    weights = None
+    if on_host:
+        sources = [(payload.quantized, payload.absmax) for _, _, payload, _ in members]
+        weights = dequantize_4bit_host(items(sources), device)
+        if weights is not None:
+            _keep_while_read(sources, device)
+    if weights is None:
+        weights = dequantize_4bit_many(items([prefetched if prefetched is not None else _upload_nf4(payload, device)
+                                              for _, _, payload, prefetched in members]))
+    for (slot, p, _, _), w in zip(members, weights):
+        _replace_param_data(p, _hand_over(w, consumers), owner=slot.owner, pname=slot.name)
 
 
 def _needs(p: torch.nn.Parameter, device: torch.device) -> bool:
@@ -568,6 +612,7 @@ def free_weights(module: torch.nn.Module) -> int:
     """Drop the device data of every staged parameter of *module* (the payloads
     stay); returns how many were dropped (``stratum/upload.py:1144-1159``)."""
     dropped = 0
+    _release_host_reads()
     for _, p in _plan(module).unique_params():
         if p.data.numel() and _staged(p) is not None:
             p.data = torch.empty(0, dtype=p.dtype, device=p.device)

@@ -467,3 +467,21 @@ def test_wrappers_refuse_operands_on_another_device():
     _on_device(dev, a=torch.empty(2, device=dev), b=None)
     with pytest.raises(ValueError, match="b is on cpu"):
         _on_device(dev, a=torch.empty(2, device=dev), b=torch.zeros(2))
+
+
+def test_dequantize_host_arguments_and_pageable_memory(L):
+    """Refused before any launch: bad arguments, and memory that no GPU can read."""
+    buf = ctypes.create_string_buffer(4096)
+    p = (ctypes.addressof(buf) + 63) // 64 * 64
+    ptrs, nulls = (ctypes.c_void_p * 1)(p), (ctypes.c_void_p * 1)(None)
+    n = (ctypes.c_int64 * 1)(128)
+    assert L.stm_nf4_dequantize_host(-1, None, None, None, 64, None, 0, None) == -1
+    assert L.stm_nf4_dequantize_host(0, None, None, None, 64, None, 0, None) == 0
+    assert L.stm_nf4_dequantize_host(1, ptrs, ptrs, n, 48, ptrs, 0, None) == -1
+    assert L.stm_nf4_dequantize_host(1, ptrs, ptrs, n, 64, ptrs, 9, None) == -1
+    assert L.stm_nf4_dequantize_host(1, nulls, ptrs, n, 64, ptrs, 0, None) == -1
+    assert L.stm_nf4_dequantize_host(1, ptrs, ptrs, (ctypes.c_int64 * 1)(-8), 64, ptrs, 0, None) == -1
+    assert L.stm_nf4_dequantize_host(1, ptrs, ptrs, (ctypes.c_int64 * 1)(12), 64, ptrs, 0, None) == -2
+    assert L.stm_nf4_dequantize_host(1, ptrs, ptrs, n, 64, ptrs, 0, None) == -2   # pageable
+    assert "pinned" in _err(L)
+    assert L.stm_event_done(None) == -1

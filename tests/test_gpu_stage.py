@@ -200,3 +200,77 @@ def test_layer_stream_mixed_nf4_and_fp16_staged(cuda):
             assert torch.equal(ga.cpu(), expect_a[i]), f"rep {rep} layer {i} NF4 weight"
             assert torch.equal(gb.cpu(), expect_b[i]), f"rep {rep} layer {i} FP16-staged weight"
         assert all(l.a.weight.numel() == 0 and l.b.weight.numel() == 0 for l in layers)
+
+
+def _host_payload(n, bs, seed, dtype=torch.float16):
+    from stratum_amd.functional import quantize_4bit
+    packed, st = quantize_4bit(seeded((n,), seed, 0.02, dtype).cuda(), blocksize=bs)
+    st.absmax, packed_host = st.absmax.cpu().pin_memory(), packed.cpu().pin_memory()
+    return packed, packed_host, st
+
+
+@pytest.mark.parametrize("bs", [64, 256])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+def test_dequantize_from_pinned_memory_is_bit_exact(cuda, bs, dtype):
+    """One group of 8, one chunk and one more, a partial block, more chunks than work-groups."""
+    from stratum_amd.functional import QuantState, dequantize_4bit, dequantize_4bit_host
+    sizes = [8, 72, 16384, 16392, 5 * 16384 + 40, 140 * 16384 + 8]
+    loads = [_host_payload(n, bs, i, dtype) for i, n in enumerate(sizes)]
+    got = dequantize_4bit_host([(host, st) for _, host, st in loads], torch.device("cuda", 0))
+    for (packed, _, st), w in zip(loads, got):
+        want = dequantize_4bit(packed, QuantState(absmax=st.absmax.cuda(), shape=st.shape, blocksize=bs, dtype=dtype))
+        assert torch.equal(w, want)
+
+
+def test_dequantize_from_host_memory_takes_only_whole_pinned_payloads(cuda):
+    from stratum_amd.functional import QuantState, dequantize_4bit_host
+    dev = torch.device("cuda", 0)
+    _, host, st = _host_payload(4096, 64, 1)
+    assert dequantize_4bit_host([(host, st)], dev) is not None
+    assert dequantize_4bit_host([(host.clone(), st)], dev) is None                 # pageable codes
+    pageable = QuantState(absmax=st.absmax.clone(), shape=st.shape, dtype=st.dtype)
+    assert dequantize_4bit_host([(host, pageable)], dev) is None                   # pageable absmax
+    assert dequantize_4bit_host([(host, st)] * 33, dev) is None
+    odd = QuantState(absmax=st.absmax, shape=(4095,), dtype=st.dtype)
+    assert dequantize_4bit_host([(host, odd)], dev) is None                        # not whole groups of 8
+    assert dequantize_4bit_host([(host[1:], QuantState(absmax=st.absmax, shape=(4088,), dtype=st.dtype))], dev) is None
+
+
+def test_a_payload_dropped_after_ensure_weights_is_still_read_whole(cuda):
+    """The launch waits behind other work; meanwhile the module and its payload go
+    and the host takes pinned memory of the same sizes and fills it."""
+    import stratum_amd.upload as U
+    w16 = seeded((1024, 512), 5, 0.02, torch.float16)
+    layer = nn.Module()
+    layer.weight = nn.Parameter(w16.clone(), requires_grad=False)
+    U.prepare_nf4(layer, verbose=False)
+    nbytes = getattr(layer.weight, U.NF4_ATTR).quantized.numel()
+    torch.cuda.synchronize()
+    torch.cuda._sleep(200_000_000)
+    U.ensure_weights(layer, 0)
+    w = layer.weight.data
+    del layer
+    taken = [torch.empty(nbytes, dtype=torch.uint8, pin_memory=True).fill_(0xFF) for _ in range(4)]
+    assert torch.equal(w.cpu().view(torch.int16), oracle_bits(w16))
+    U._release_host_reads()
+    assert not U._host_reads and len(taken) == 4
+
+
+def test_ensure_weights_inside_a_captured_graph_reads_the_payload_on_each_replay(cuda):
+    import stratum_amd.upload as U
+    layer = _two_layers()[0]
+    U.ensure_weights(layer, 0)
+    want = [p.detach().clone() for p in layer.parameters()]
+    U.free_weights(layer)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        U.ensure_weights(layer, 0, consumers=[])
+        held = [p.data for p in layer.parameters()]
+    for _ in range(3):
+        for h in held:
+            if h.is_cuda:
+                h.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(h, w) for h, w in zip(held, want) if h.dim() == 2)
