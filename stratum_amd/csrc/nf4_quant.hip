@@ -543,7 +543,7 @@ __global__ __launch_bounds__(256) void k_dequantize_many(DequantMany m) {
 // other streams. A layer of seven projections (8.8 MB packed): 165 us, against
 // 315 us as 14 uploads and a batched dequantize.
 template <int DT, int U>
-__global__ __launch_bounds__(256) void k_dequantize_host(DequantMany m) {
+__global__ __launch_bounds__(256) void k_dequantize_many_host(DequantMany m) {
     __shared__ float2 lut[256];
     fill_byte_lut(lut);
     const int64_t chunks = m.first_wg[m.count];
@@ -695,7 +695,7 @@ static void dequant_host_launch(DequantMany& m, hipStream_t stream) {
     m.first_wg[0] = 0;
     for (int t = 0; t < m.count; ++t) m.first_wg[t + 1] = m.first_wg[t] + (m.ngroups[t] + U * 256 - 1) / (U * 256);
     const int64_t chunks = m.first_wg[m.count];
-    hipLaunchKernelGGL((k_dequantize_host<DT, U>), dim3((unsigned)(chunks < kHostWgs ? chunks : kHostWgs)), dim3(256),
+    hipLaunchKernelGGL((k_dequantize_many_host<DT, U>), dim3((unsigned)(chunks < kHostWgs ? chunks : kHostWgs)), dim3(256),
                        0, stream, m);
 }
 
