@@ -427,6 +427,7 @@ int stm_nf4_grouped_gemm_fwd(const void* X, const uint8_t* packed, const float* 
     GemmArgs g{};
     g.a = X; g.packed = packed; g.absmax = absmax; g.out = Y; g.M = max_rows; g.N = N; g.K = K;
     g.blocksize = blocksize; g.offsets = offsets; g.num_groups = num_experts;
+    for (int e = 0; host_offsets && e < num_experts; ++e) g.hits += host_offsets[e + 1] > host_offsets[e];
     g.group_bm = host_offsets ? grouped_tile_rows(host_offsets, num_experts) : 0;
     g.stream_out = host_offsets && (int64_t)host_offsets[num_experts] * N * 2 >= kStreamOutBytes;
     return launch_gemm_fwd(g, dtype, (hipStream_t)stream);

@@ -152,6 +152,39 @@ __device__ __forceinline__ Group group_of(const GemmArgs& g, int e) {
     return r;
 }
 
+// The experts that have rows, in order: a walk over the offsets, 64 experts at a
+// time (one of them per lane), that only moves forward. Every lane of the wave
+// takes part. An expert's row range comes out of the walk's registers, with no
+// second round trip to memory.
+struct HitWalk {
+    int seen = 0;            // experts with rows before experts e0 .. e0 + 63
+    int e0 = -64;
+    uint64_t with_rows = 0;  // those of e0 .. e0 + 63, a bit each
+    int first, end;          // this lane's expert: its row range
+
+    // Expert number q (from 0) among those with rows; false past the last. q never decreases.
+    __device__ __forceinline__ bool find(const GemmArgs& g, int q, int lane, Group& r) {
+        while (q - seen >= __popcll(with_rows)) {
+            seen += __popcll(with_rows);
+            e0 += 64;
+            if (e0 >= g.num_groups) return false;
+            const int e = e0 + lane < g.num_groups ? e0 + lane : g.num_groups - 1;
+            first = g.offsets[e];
+            end = g.offsets[e + 1];
+            with_rows = __ballot(e0 + lane < g.num_groups && end > first);
+        }
+        const int below = __builtin_amdgcn_mbcnt_hi((uint32_t)(with_rows >> 32),
+                                                    __builtin_amdgcn_mbcnt_lo((uint32_t)with_rows, 0));
+        const int at = __builtin_ctzll(__ballot((with_rows >> lane & 1) && below == q - seen));
+        const int64_t e = e0 + at, wnum = g.N * g.K;
+        r.row0 = __builtin_amdgcn_readlane(first, at);
+        r.rows = __builtin_amdgcn_readlane(end, at) - r.row0;
+        r.packed = g.packed + e * (wnum / 2);
+        r.absmax = g.absmax + e * (wnum / g.blocksize);
+        return true;
+    }
+};
+
 // Tile order: work-groups are dispatched round-robin over the 8 XCDs, so ids
 // i, i + 8, i + 16, ... share an L2. Give each XCD a contiguous run of tiles and
 // walk them GROUP_M activation tiles at a time so concurrently running tiles on
@@ -1893,59 +1926,61 @@ __global__ __launch_bounds__((64 * GvCfg<MB, GK>::WAVES)) void k_gemv_fwd(GemmAr
     const int nfl = (C::GK >> bshift) > 0 ? (C::GK >> bshift) : 1;  // absmax per row per group
     const int64_t kblocks = K >> bshift;
     const int ngroups = (int)((K + C::GK - 1) / C::GK);
-    // GROUPED: expert blockIdx.y (one reduction range): its rows from the
-    // offsets, at most g.M (the caller's bound, at most 16 MB rows), its
-    // weight and its output rows; a work-group of an empty expert leaves
-    // before any barrier
-    int64_t M = g.M;
-    const uint16_t* xa = reinterpret_cast<const uint16_t*>(g.a);
-    const uint8_t* wpk = g.packed;
-    const float* wab = g.absmax;
+    // what the copies and the stores of a work item need (an item: this
+    // work-group's block of weight rows over groups [g_begin, g_end))
+    int64_t M = g.M, nw0 = (int64_t)blockIdx.x * C::ROWS + wave * C::RW;  // activation rows, this wave's first weight row
     uint16_t* yo = reinterpret_cast<uint16_t*>(g.out);
-    int z = blockIdx.y;
-    if constexpr (GROUPED) {
-        const Group gr = group_of(g, (int)blockIdx.y);
-        M = gr.rows < 0 ? 0 : gr.rows < g.M ? gr.rows : g.M;
-        if (M <= 0) return;
-        xa += gr.row0 * K;
-        yo += gr.row0 * N;
-        wpk = gr.packed;
-        wab = gr.absmax;
-        z = 0;
-    }
+    const int z = GROUPED ? 0 : blockIdx.y;
     const int g_begin = z * groups_per_split;
     const int g_end = g_begin + groups_per_split < ngroups ? g_begin + groups_per_split : ngroups;
-    const int64_t nw0 = (int64_t)blockIdx.x * C::ROWS + wave * C::RW;  // this wave's first weight row
 
     // copy sources (per lane; group offsets added per copy): weight copy i
     // covers rows 64 / PW i + lane / PW, slot lane % PW of each
     constexpr int PW = C::PW, WC = C::RW * PW / 64;
     auto wslot_piece = [](int row, int slot) { return slot ^ ((row >> C::WSH) & (PW - 1)); };
-    const uint8_t* wsrc[WC];
-#pragma unroll
-    for (int i = 0; i < WC; ++i) {
-        const int row = 64 / PW * i + lane / PW;
-        const int64_t n = nw0 + row < N ? nw0 + row : N - 1;
-        wsrc[i] = wpk + n * (K / 2) + 16 * wslot_piece(row, lane % PW);
-    }
     const int a_rows_per_copy = 64 / nfl, a_copies = (C::RW * nfl + 63) / 64;  // <= R
-    const float* asrc[R];
-#pragma unroll
-    for (int i = 0; i < R; ++i) {
-        const int64_t n0 = nw0 + lane / nfl + i * a_rows_per_copy;
-        asrc[i] = wab + (n0 < N ? n0 : N - 1) * kblocks;
-    }
     const int aj = lane % nfl;
     // activations: XR PX / 64 copies of 64 / PX rows each, copy ix by wave ix % WAVES
     constexpr int PX = C::PX, XI = C::XR * PX / 64, XC = (XI + WAVES - 1) / WAVES;
+    const uint8_t* wsrc[WC];
+    const float* asrc[R];
     const uint16_t* xsrc[XC];
     int xpiece[XC];
+    auto aim = [&](const uint16_t* xa, const uint8_t* wpk, const float* wab) {
 #pragma unroll
-    for (int j = 0; j < XC; ++j) {
-        const int xm = 64 / PX * (wave + j * WAVES) + lane / PX;  // activation row this lane copies
-        xsrc[j] = xa + (xm < M ? xm : M - 1) * K;
-        xpiece[j] = (lane % PX) ^ (xm & 15);
-    }
+        for (int i = 0; i < WC; ++i) {
+            const int row = 64 / PW * i + lane / PW;
+            const int64_t n = nw0 + row < N ? nw0 + row : N - 1;
+            wsrc[i] = wpk + n * (K / 2) + 16 * wslot_piece(row, lane % PW);
+        }
+#pragma unroll
+        for (int i = 0; i < R; ++i) {
+            const int64_t n0 = nw0 + lane / nfl + i * a_rows_per_copy;
+            asrc[i] = wab + (n0 < N ? n0 : N - 1) * kblocks;
+        }
+#pragma unroll
+        for (int j = 0; j < XC; ++j) {
+            const int xm = 64 / PX * (wave + j * WAVES) + lane / PX;  // activation row this lane copies
+            xsrc[j] = xa + (xm < M ? xm : M - 1) * K;
+            xpiece[j] = (lane % PX) ^ (xm & 15);
+        }
+    };
+
+    // GROUPED: the items are (expert with rows, block of weight rows), expert
+    // by expert; this work-group runs items blockIdx.x, + gridDim.x, ...
+    const int blocks = (int)((N + C::ROWS - 1) / C::ROWS);
+    int item = blockIdx.x;
+    HitWalk walk;
+    auto next_item = [&]() {  // aims at item `item`; false past the last
+        Group gr;
+        if (!walk.find(g, item / blocks, lane, gr)) return false;
+        M = gr.rows < g.M ? gr.rows : g.M;  // at most the caller's bound, at most 16 MB rows
+        nw0 = (int64_t)(item % blocks) * C::ROWS + wave * C::RW;
+        yo = reinterpret_cast<uint16_t*>(g.out) + gr.row0 * N;
+        aim(reinterpret_cast<const uint16_t*>(g.a) + gr.row0 * K, gr.packed, gr.absmax);
+        item += gridDim.x;
+        return true;
+    };
 
     auto uniform = [](uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane(v); };
     auto copy_group = [&](int grp, int buf) {
@@ -2042,48 +2077,86 @@ __global__ __launch_bounds__((64 * GvCfg<MB, GK>::WAVES)) void k_gemv_fwd(GemmAr
         }
     };
 
-    if (g_begin < g_end) copy_group(g_begin, 0);  // in flight while the level table is filled
-    fill_lut_rw<64 * WAVES>(lut_all, tid);
-    wait_vmem();
-    __syncthreads();  // level table and group g_begin ready
-    for (int grp = g_begin; grp < g_end; ++grp) {
-        const int buf = (grp - g_begin) & 1;
-        if (grp + 1 < g_end) copy_group(grp + 1, buf ^ 1);
-        if ((int64_t)(grp + 1) * C::GK > K)
-            compute(buf, grp, std::true_type());
-        else
-            compute(buf, grp, std::false_type());
-        wait_vmem();
-        __syncthreads();  // group grp + 1 landed; every wave is done reading this buffer
-    }
-
-    // C[4 h + i][r] of tile t, block mb: weight row nw0 + 16 t + 4 h + i, activation row 16 mb + r
-    const uint16_t* bias = reinterpret_cast<const uint16_t*>(g.bias);
+    // C[4 h + i][r] of tile t, block mb: weight row n0 + 16 t + 4 h + i, activation row 16 mb + r
+    auto store = [&](const f32x4_t (&v4)[R][MB], int64_t rows, int64_t n0, uint16_t* y) {
+        const uint16_t* bias = reinterpret_cast<const uint16_t*>(g.bias);
 #pragma unroll
-    for (int t = 0; t < R; ++t)
+        for (int t = 0; t < R; ++t)
 #pragma unroll
-        for (int mb = 0; mb < MB; ++mb) {
-            const int64_t m = 16 * mb + r;
-            const int64_t nc = nw0 + 16 * t + 4 * h;
-            if (m >= M || nc >= N) continue;  // N % 8 == 0: all four columns valid
-            if (g.splits > 1) {
-                *reinterpret_cast<float4*>(g.partial + (int64_t)z * M * N + m * N + nc) =
-                    make_float4(acc[t][mb][0], acc[t][mb][1], acc[t][mb][2], acc[t][mb][3]);
-            } else {
-                float v[4] = {acc[t][mb][0], acc[t][mb][1], acc[t][mb][2], acc[t][mb][3]};
-                if (bias) {  // 2-byte aligned: four 16-bit loads, issued together
-                    uint16_t bb[4];
+            for (int mb = 0; mb < MB; ++mb) {
+                const int64_t m = 16 * mb + r;
+                const int64_t nc = n0 + 16 * t + 4 * h;
+                if (m >= rows || nc >= N) continue;  // N % 8 == 0: all four columns valid
+                if (!GROUPED && g.splits > 1) {
+                    *reinterpret_cast<float4*>(g.partial + (int64_t)z * rows * N + m * N + nc) =
+                        make_float4(v4[t][mb][0], v4[t][mb][1], v4[t][mb][2], v4[t][mb][3]);
+                } else {
+                    float v[4] = {v4[t][mb][0], v4[t][mb][1], v4[t][mb][2], v4[t][mb][3]};
+                    if (!GROUPED && bias) {  // 2-byte aligned: four 16-bit loads, issued together
+                        uint16_t bb[4];
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) bb[i] = bias[nc + i];
+                        for (int i = 0; i < 4; ++i) bb[i] = bias[nc + i];
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) v[i] += Tr::to_f32(bb[i]);
+                        for (int i = 0; i < 4; ++i) v[i] += Tr::to_f32(bb[i]);
+                    }
+                    uint2 pk;
+                    pk.x = Tr::pack2(v[0], v[1]);
+                    pk.y = Tr::pack2(v[2], v[3]);
+                    *reinterpret_cast<uint2*>(y + m * N + nc) = pk;
                 }
-                uint2 pk;
-                pk.x = Tr::pack2(v[0], v[1]);
-                pk.y = Tr::pack2(v[2], v[3]);
-                *reinterpret_cast<uint2*>(yo + m * N + nc) = pk;
             }
+    };
+
+    if constexpr (GROUPED) {
+        // One work-group per CU over all items, one stream of groups across
+        // them: the level table is filled once, and the first group of the
+        // next item is copied while the last group of this one is computed.
+        if (!next_item()) return;  // every wave alike, before any barrier
+        const int steps = ngroups > 0 ? ngroups : 1;  // K = 0: one group with nothing in it, zeros stored
+        if (K > 0) copy_group(0, 0);
+        fill_lut_rw<64 * WAVES>(lut_all, tid);
+        wait_vmem();
+        __syncthreads();
+        bool more = true;
+        int buf = 0;
+        while (more) {
+            const int64_t rows = M, n0 = nw0;
+            uint16_t* y = yo;
+            for (int grp = 0; grp < steps; ++grp, buf ^= 1) {
+                const bool last = grp + 1 == steps;
+                if (last) more = next_item();
+                if (more && K > 0) copy_group(last ? 0 : grp + 1, buf ^ 1);
+                if ((int64_t)(grp + 1) * C::GK > K)
+                    compute(buf, grp, std::true_type());
+                else
+                    compute(buf, grp, std::false_type());
+                wait_vmem();
+                __syncthreads();  // the next group landed; every wave is done reading this buffer
+            }
+            store(acc, rows, n0, y);  // awaited a group later, under that group's math
+#pragma unroll
+            for (int t = 0; t < R; ++t)
+#pragma unroll
+                for (int mb = 0; mb < MB; ++mb) acc[t][mb] = f32x4_t{0.f, 0.f, 0.f, 0.f};
         }
+    } else {
+        aim(reinterpret_cast<const uint16_t*>(g.a), g.packed, g.absmax);
+        if (g_begin < g_end) copy_group(g_begin, 0);  // in flight while the level table is filled
+        fill_lut_rw<64 * WAVES>(lut_all, tid);
+        wait_vmem();
+        __syncthreads();  // level table and group g_begin ready
+        for (int grp = g_begin; grp < g_end; ++grp) {
+            const int buf = (grp - g_begin) & 1;
+            if (grp + 1 < g_end) copy_group(grp + 1, buf ^ 1);
+            if ((int64_t)(grp + 1) * C::GK > K)
+                compute(buf, grp, std::true_type());
+            else
+                compute(buf, grp, std::false_type());
+            wait_vmem();
+            __syncthreads();  // group grp + 1 landed; every wave is done reading this buffer
+        }
+        store(acc, M, nw0, yo);
+    }
 }
 
 // Small-M forward without a split reduction (up to 16 activation rows). A
@@ -2113,7 +2186,7 @@ struct GkCfg {
     static_assert(8 * TW * 64 * 16 <= kW, "the slice sums fit the weight buffer");
 };
 
-template <typename Tr, int T, int TW, int XR>
+template <typename Tr, int T, int TW, int XR, bool GROUPED = false>
 __global__ __launch_bounds__(512) void k_gemv_ks(GemmArgs g) {
     using C = GkCfg<T, TW, XR>;
     constexpr int S = C::S, ROWS = C::ROWS, P = C::P;
@@ -2127,13 +2200,18 @@ __global__ __launch_bounds__(512) void k_gemv_ks(GemmArgs g) {
     auto ba = [&](int b) { return reinterpret_cast<float*>(smem + C::kLut + b * C::kBuf + C::kW); };
     auto bx = [&](int b) { return reinterpret_cast<uint4*>(smem + C::kLut + b * C::kBuf + C::kW + C::kA); };
 
-    const int64_t K = g.K, N = g.N, M = g.M;
+    const int64_t K = g.K, N = g.N;
     const int bshift = 31 - __builtin_clz(g.blocksize);
     const int nfl = (GV_GK >> bshift) > 0 ? (GV_GK >> bshift) : 1;  // absmax per row per group
     const int64_t kblocks = K >> bshift;
     const int ngroups = (int)((K + GV_GK - 1) / GV_GK);
     const int steps = (ngroups + S - 1) / S;
-    const int64_t n0 = (int64_t)blockIdx.x * ROWS;
+    int64_t M = g.M, n0 = (int64_t)blockIdx.x * ROWS;
+    const uint16_t* xa = reinterpret_cast<const uint16_t*>(g.a);
+    const uint8_t* wpk = g.packed;
+    const float* wab = g.absmax;
+    uint16_t* yo = reinterpret_cast<uint16_t*>(g.out);
+    auto body = [&]() {
     auto uniform = [](uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane(v); };
 
     // copy sources, per thread. Packed weight: row-slice q = 16 TW wave + 8 i +
@@ -2146,7 +2224,7 @@ __global__ __launch_bounds__(512) void k_gemv_ks(GemmArgs g) {
         wsl[i] = q / ROWS;
         wpiece[i] = (lane & 7) ^ ((row >> 1) & 7);
         const int64_t n = n0 + row < N ? n0 + row : N - 1;
-        wsrc[i] = g.packed + n * (K / 2) + 16 * wpiece[i];
+        wsrc[i] = wpk + n * (K / 2) + 16 * wpiece[i];
     }
     // absmax: thread tid copies entries e = tid + 512 i = (row-slice q) nfl + j
     // of RS nfl (whole waves: 128 TW nfl entries)
@@ -2159,7 +2237,7 @@ __global__ __launch_bounds__(512) void k_gemv_ks(GemmArgs g) {
         asl[i] = q / ROWS;
         aj[i] = e % nfl;
         const int64_t n = n0 + q % ROWS < N ? n0 + q % ROWS : N - 1;
-        asrc[i] = g.absmax + n * kblocks;
+        asrc[i] = wab + n * kblocks;
     }
     // activations: piece p = tid + 512 i of S x XR x 32 (row xr of slice xs)
     const uint16_t* xsrc[2];
@@ -2171,7 +2249,7 @@ __global__ __launch_bounds__(512) void k_gemv_ks(GemmArgs g) {
         xsl[i] = p / (XR * 32);
         xon[i] = p < S * XR * 32 && xr < M;
         xpiece[i] = (p % 32) ^ (xr & 15);
-        xsrc[i] = reinterpret_cast<const uint16_t*>(g.a) + (xr < M ? xr : 0) * K;
+        xsrc[i] = xa + (xr < M ? xr : 0) * K;
     }
 
     auto copy_step = [&](int j, int b) {
@@ -2295,7 +2373,7 @@ __global__ __launch_bounds__(512) void k_gemv_ks(GemmArgs g) {
         red[(s * T + t0 + u) * 64 + lane] = make_float4(acc[u][0], acc[u][1], acc[u][2], acc[u][3]);
     __syncthreads();
     if (s != 0) return;
-    const int R = g.lora_rank;
+    const int R = GROUPED ? 0 : g.lora_rank;
     const uint16_t* bias = reinterpret_cast<const uint16_t*>(g.bias);
 #pragma unroll
     for (int u = 0; u < TW; ++u) {
@@ -2333,7 +2411,7 @@ __global__ __launch_bounds__(512) void k_gemv_ks(GemmArgs g) {
 #pragma unroll
             for (int i = 0; i < 4; ++i) v[i] += l[i];
         }
-        if (bias) {
+        if (!GROUPED && bias) {
             uint16_t bb[4];
 #pragma unroll
             for (int i = 0; i < 4; ++i) bb[i] = bias[nc + i];
@@ -2343,7 +2421,29 @@ __global__ __launch_bounds__(512) void k_gemv_ks(GemmArgs g) {
         uint2 pk;
         pk.x = Tr::pack2(v[0], v[1]);
         pk.y = Tr::pack2(v[2], v[3]);
-        *reinterpret_cast<uint2*>(reinterpret_cast<uint16_t*>(g.out) + m * N + nc) = pk;
+        *reinterpret_cast<uint2*>(yo + m * N + nc) = pk;
+    }
+    };
+    if constexpr (GROUPED) {
+        // items (expert with rows, block of weight rows), expert by expert, one
+        // per work-group (more only where the host counted fewer such experts
+        // than the offsets hold)
+        const int blocks = (int)((N + ROWS - 1) / ROWS);
+        HitWalk walk;
+        Group gr;
+        for (int item = blockIdx.x;; item += gridDim.x) {
+            if (!walk.find(g, item / blocks, lane, gr)) return;  // every wave alike
+            M = gr.rows < g.M ? gr.rows : g.M;  // at most the caller's bound, at most XR
+            n0 = (int64_t)(item % blocks) * ROWS;
+            xa = reinterpret_cast<const uint16_t*>(g.a) + gr.row0 * K;
+            yo = reinterpret_cast<uint16_t*>(g.out) + gr.row0 * N;
+            wpk = gr.packed;
+            wab = gr.absmax;
+            body();
+            __syncthreads();  // LDS is free for the next item
+        }
+    } else {
+        body();
     }
 }
 
@@ -3188,35 +3288,48 @@ int64_t gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, bool backward, int
 // (event-timed, µs): K <= 4096 faster, e.g. [4096,4096] M = 8 12.2 -> 10.0,
 // [2048,4096] M = 1 10.8 -> 7.6, [8192,1024] M = 12 10.5 -> 7.6, [8192,4096]
 // M = 16 14.3 / 14.5; K >= 11008 slower ([4096,14336] M = 8 17.5 / 20.2).
+static const int kKsConfigs[][3] = {{1, 1, 4}, {2, 1, 8}, {4, 1, 16}, {8, 1, 16}, {4, 2, 4}};  // T, TW, XR
+
+// Work-groups of one configuration and its time in tile-groups per wave.
+static double gemv_ks_time(const int (&c)[3], int64_t hits, int64_t N, int64_t K, int64_t cus, int64_t* blocks) {
+    const int T = c[0], TW = c[1], S = 8 * TW / T;
+    const int64_t groups = (K + GV_GK - 1) / GV_GK;
+    *blocks = hits * ((N + 16 * T - 1) / (16 * T));
+    const int64_t rounds = (*blocks + cus - 1) / cus;
+    return (double)rounds * (1.0 + (double)((groups + S - 1) / S) * TW * (TW == 1 ? 1.25 : 1.0));
+}
+
 int gemv_ks_config(int64_t M, int64_t N, int64_t K) {
     if (!STM_GEMV_KS || M < 1 || M > 16) return 0;
-    static const int cfgs[][3] = {{1, 1, 4}, {2, 1, 8}, {4, 1, 16}, {8, 1, 16}, {4, 2, 4}};
     const int64_t groups = (K + GV_GK - 1) / GV_GK, cus = device_cus();
     int best = 0;
     for (int pass = 0; pass < 2 && !best; ++pass) {
         if (pass == 1 && groups > 16) break;
         double best_t = 1e30;
-        for (const auto& c : cfgs) {
-            const int T = c[0], TW = c[1], XR = c[2], S = 8 * TW / T;
-            if (M > XR) continue;
-            const int64_t blocks = (N + 16 * T - 1) / (16 * T);
+        for (const auto& c : kKsConfigs) {
+            if (M > c[2]) continue;
+            int64_t blocks;
+            const double t = gemv_ks_time(c, 1, N, K, cus, &blocks);
             if (pass == 0 ? blocks * 4 < cus * 3 : blocks * 2 < cus) continue;
-            const int64_t rounds = (blocks + cus - 1) / cus;
-            const double t = (double)rounds * (1.0 + (double)((groups + S - 1) / S) * TW * (TW == 1 ? 1.25 : 1.0));
-            if (t < best_t) best_t = t, best = T | TW << 4 | XR << 8;
+            if (t < best_t) best_t = t, best = c[0] | c[1] << 4 | c[2] << 8;
         }
     }
     return best;
 }
 int gemv_ks_tiles(int64_t M, int64_t N, int64_t K) { return gemv_ks_config(M, N, K); }
 
-int launch_gemv_ks(const GemmArgs& g, int cfg, int dtype, hipStream_t stream) {
+// hits > 0: a grouped launch over that many experts with rows.
+int launch_gemv_ks(const GemmArgs& g, int cfg, int dtype, hipStream_t stream, int hits = 0) {
     const int T = cfg & 15;
-    const dim3 grid((unsigned)((g.N + 16 * T - 1) / (16 * T))), block(512);
-#define STM_KS_LAUNCH(TT, TW, XR)                                                           \
-    if (dtype == STM_BF16)                                                                  \
-        hipLaunchKernelGGL((k_gemv_ks<BF16, TT, TW, XR>), grid, block, 0, stream, g);       \
-    else                                                                                    \
+    const dim3 grid((unsigned)((g.N + 16 * T - 1) / (16 * T) * (hits ? hits : 1))), block(512);
+#define STM_KS_LAUNCH(TT, TW, XR)                                                                 \
+    if (dtype == STM_BF16 && hits)                                                                \
+        hipLaunchKernelGGL((k_gemv_ks<BF16, TT, TW, XR, true>), grid, block, 0, stream, g);       \
+    else if (dtype == STM_BF16)                                                                   \
+        hipLaunchKernelGGL((k_gemv_ks<BF16, TT, TW, XR>), grid, block, 0, stream, g);             \
+    else if (hits)                                                                                \
+        hipLaunchKernelGGL((k_gemv_ks<F16, TT, TW, XR, true>), grid, block, 0, stream, g);        \
+    else                                                                                          \
         hipLaunchKernelGGL((k_gemv_ks<F16, TT, TW, XR>), grid, block, 0, stream, g);
     switch (cfg) {
         case 1 | 1 << 4 | 4 << 8: STM_KS_LAUNCH(1, 1, 4) break;
@@ -3230,6 +3343,27 @@ int launch_gemv_ks(const GemmArgs& g, int cfg, int dtype, hipStream_t stream) {
     return check_launch("gemm_fwd (small M, one launch)");
 }
 
+// Split-free configuration for a grouped forward over `hits` experts with rows
+// (0: unknown) of at most M rows each, or 0 where one work-group per CU over
+// whole-reduction items (k_gemv_fwd) is estimated faster, in the same unit:
+// two tile-groups per group, the fixed cost once. Few experts leave that
+// kernel's 256-row items on few CUs ([1536, 2048] over 8 of 128 experts: 17.7
+// against 8.0 us); many pay the split-free kernel's fixed cost once per
+// work-group, for which its estimate counts 1.3 times (30 experts: 20.5
+// against 23.0 us).
+int gemv_ks_grouped_config(int64_t M, int hits, int64_t N, int64_t K) {
+    if (!STM_GEMV_KS || M < 1 || M > 16 || hits < 1) return 0;
+    const int64_t cus = device_cus(), items = hits * ((N + GvCfg<1, 256>::ROWS - 1) / GvCfg<1, 256>::ROWS);
+    double best_t = 1.0 + 2.0 * (double)((items + cus - 1) / cus) * (double)((K + GV_GK - 1) / GV_GK);
+    int best = 0;
+    for (const auto& c : kKsConfigs) {
+        int64_t blocks;
+        const double t = gemv_ks_time(c, hits, N, K, cus, &blocks);
+        if (M <= c[2] && 1.3 * t < best_t) best_t = 1.3 * t, best = c[0] | c[1] << 4 | c[2] << 8;
+    }
+    return best;
+}
+
 // 1: grouped forwards whose experts hold at most 64 rows run the
 // weight-streaming kernel.
 #ifndef STM_GEMV_GROUPED
@@ -3237,17 +3371,23 @@ int launch_gemv_ks(const GemmArgs& g, int cfg, int dtype, hipStream_t stream) {
 #endif
 
 // Grouped forward with at most 64 rows per expert (the caller's max_rows, so
-// decode-sized MoE batches): one work-group per (block of weight rows,
-// expert), each over the whole reduction (no partials, no workspace); an
-// empty expert's work-groups leave at once. The tile path would run 192- or
-// 256-row tiles of MFMAs for each expert's few rows.
+// decode-sized MoE batches): one work-group per CU walks the items (expert with
+// rows, block of weight rows), each over the whole reduction (no partials, no
+// workspace), or the split-free kernel for few experts. The tile path would run
+// 192- or 256-row tiles of MFMAs for each expert's few rows. Bound by the
+// dequantization (2.0-2.2 us per 256-deep group and CU). Against one work-group
+// per item, whose level table and first copies were exposed once per item and
+// whose last round left most CUs idle: [1536, 2048] and [2048, 768] over 82 of
+// 128 experts 51.0 -> 34.8 and 30.8 -> 22.1 us, over 125 experts 54.3 -> 50.3
+// and 33.4 -> 27.8 us.
 int launch_gemv_grouped(GemmArgs g, int dtype, hipStream_t stream) {
     g.splits = 1;
+    if (const int ks = gemv_ks_grouped_config(g.M, g.hits, g.N, g.K)) return launch_gemv_ks(g, ks, dtype, stream, g.hits);
 #define STM_GG_LAUNCH(MB, GKV)                                                                          \
     {                                                                                                   \
         const int ng = (int)((g.K + GKV - 1) / GKV);                                                    \
-        const dim3 grid((unsigned)((g.N + GvCfg<MB, GKV>::ROWS - 1) / GvCfg<MB, GKV>::ROWS),            \
-                        (unsigned)g.num_groups),                                                        \
+        const int64_t items = (g.N + GvCfg<MB, GKV>::ROWS - 1) / GvCfg<MB, GKV>::ROWS * g.num_groups;   \
+        const dim3 grid((unsigned)(items < device_cus() ? items : device_cus())),                       \
             block(64 * GvCfg<MB, GKV>::WAVES);                                                          \
         if (dtype == STM_BF16)                                                                          \
             hipLaunchKernelGGL((k_gemv_fwd<BF16, MB, GKV, true>), grid, block, 0, stream, g, ng);      \

@@ -33,6 +33,8 @@ struct GemmArgs {
     // Grouped forward: tile height chosen from the host's per-expert row counts
     // (grouped_tile_rows); 0 = the planner's 256-row tile.
     int group_bm;
+    // Grouped: experts with rows, from the host's offsets; 0 = not known.
+    int hits;
     // 1: the register-weight kernels write the output with non-temporal stores.
     // Set for outputs of at least kStreamOutBytes: the next kernel would not
     // find them in the 256 MB infinity cache anyway, and written back later

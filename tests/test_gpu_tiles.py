@@ -261,6 +261,9 @@ def test_grouped_call_with_one_expert_writes_only_its_rows(cuda, backward):
     ([33, 64, 0, 2, 48, 40, 1], 264, 1536, 256, None),     # 33-64 rows, blocksize 256 (a group is half a block)
     ([9] * 40, 136, 512, 512, None),                       # 40 experts, blocksize 512
     ([40, 0, 33, 7], 264, 576, 64, None),                  # 33-48 rows: the 48-row layout
+    ([1, 4, 0, 3] * 70, 264, 320, 64, None),               # 420 items over 256 work-groups, walked over 280 experts
+    ([0] * 130 + [2] + [0] * 70 + [5], 1288, 1088, 64, None),  # two experts with rows among 202: the split-free kernel
+    ([16, 0, 1], 1032, 2176, 128, None),                   # the same, 16 rows, more groups than slices
     ([1, 0, 3, 2], 264, 576, 64, 64),                      # max_rows 64 (a bound) over 0-3 rows: the 64-row layout
 ])
 def test_grouped_forward_small_rows_per_expert(cuda, monkeypatch, dtype, counts, N, K, bs, max_rows):
@@ -291,6 +294,29 @@ def test_grouped_forward_small_rows_per_expert(cuda, monkeypatch, dtype, counts,
     set_tile(monkeypatch, "big")
     yt = nf4_grouped_gemm(x, q, a, off.to(cuda), (N, K), bs, max_rows=max_rows)
     assert rel(y, yt) <= TOL[dtype] / 4
+
+
+@pytest.mark.parametrize("host_counts", [[0, 4, 0, 0, 0, 0], [4, 4, 4, 4, 4, 4], None])
+def test_grouped_small_rows_follow_the_device_offsets(cuda, host_counts):
+    """The host's copy of the offsets sizes the launch (here: fewer or more experts
+    with rows than there are, or unknown); the rows come from the device's."""
+    from stratum_amd import _lib
+    from stratum_amd.functional import _gemm_dtype, nf4_grouped_gemm, quantize_4bit
+    dtype, counts, N, K = torch.bfloat16, [4, 1, 0, 2, 3, 4], 1032, 576
+    packed, st = quantize_4bit(seeded((6, N, K), 83, 0.02, torch.float16).to(cuda))
+    offsets = torch.tensor(np.concatenate([[0], np.cumsum(counts)]), dtype=torch.int32)
+    x = seeded((14, K), 84, 1.0, dtype).to(cuda)
+    want = nf4_grouped_gemm(x, packed, st.absmax, offsets, (N, K))
+    y = torch.full((14, N), float("nan"), dtype=dtype, device=cuda)
+    host = None if host_counts is None else torch.tensor(np.concatenate([[0], np.cumsum(host_counts)]), dtype=torch.int32)
+    dev_off = offsets.to(cuda)
+    rc = _lib.lib().stm_nf4_grouped_gemm_fwd(
+        x.data_ptr(), packed.data_ptr(), st.absmax.data_ptr(), dev_off.data_ptr(),
+        host.data_ptr() if host is not None else None, 6, 4, y.data_ptr(), N, K, 64, _gemm_dtype(x),
+        _lib.stream_handle(cuda))
+    assert rc == 0, _lib.lib().stm_last_error()
+    torch.cuda.synchronize()
+    assert rel(y, want) <= TOL[dtype] / 4  # another slicing of the fp32 sums
 
 
 @pytest.mark.parametrize("tile", ["big", "big8", "mid", "small"])
