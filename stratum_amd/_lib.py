@@ -8,6 +8,7 @@ There is no fallback: if the library is missing every call raises.
 
 from __future__ import annotations
 
+import contextlib
 import ctypes
 import os
 import threading
@@ -118,6 +119,20 @@ def dtype_tag(dtype: torch.dtype) -> int:
     raise ValueError(f"unsupported dtype {dtype} (expected float16, bfloat16 or float32)")
 
 
+def _index(device: torch.device) -> int:
+    return torch.cuda.current_device() if device.index is None else device.index
+
+
 def stream_handle(device: torch.device) -> int:
-    """hipStream_t of torch's current stream on *device*."""
-    return torch.cuda.current_stream(device).cuda_stream
+    """hipStream_t of torch's current stream on *device* (the handle alone: a
+    ``torch.cuda.Stream`` object costs 1.7 us more)."""
+    return torch._C._cuda_getCurrentRawStream(_index(device))
+
+
+_SAME_DEVICE = contextlib.nullcontext()
+
+
+def device_guard(device: torch.device):
+    """``torch.cuda.device(device)``, or nothing where it is the current device
+    already (every call of a one-process-per-GPU program: 1.2 us each)."""
+    return _SAME_DEVICE if torch.cuda.current_device() == device.index else torch.cuda.device(device)

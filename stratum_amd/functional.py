@@ -17,12 +17,25 @@ device).
 
 from __future__ import annotations
 
+import functools
 from collections import OrderedDict
 from typing import Optional, Sequence
 
 import torch
 
 from . import _lib
+
+def _no_grad(fn):
+    """``torch.no_grad()`` for a function that is mostly called with gradients off
+    (inside an autograd function, in decoding), where it costs nothing."""
+    @functools.wraps(fn)
+    def call(*args, **kwargs):
+        if not torch.is_grad_enabled():
+            return fn(*args, **kwargs)
+        with torch.no_grad():
+            return fn(*args, **kwargs)
+    return call
+
 
 # NF4 levels (QLoRA, arXiv 2305.14314 App. E); the fp32 table bitsandbytes
 # returns from get_4bit_type("nf4") and the reference stores in NF4Payload.code.
@@ -106,6 +119,11 @@ def _gpu_device(t: torch.Tensor) -> torch.device:
     return torch.device("cuda", torch.cuda.current_device())
 
 
+def _rows(t: torch.Tensor, cols: int) -> torch.Tensor:
+    """*t* as [rows, cols]."""
+    return t if t.dim() == 2 else t.reshape(-1, cols)
+
+
 def _aligned(t: torch.Tensor, a: int = 16) -> torch.Tensor:
     t = t.contiguous()
     if t.numel() and t.data_ptr() % a:
@@ -138,7 +156,7 @@ def _out_buffer(out: Optional[torch.Tensor], shape, dtype, device) -> torch.Tens
     return out.view(shape)
 
 
-@torch.no_grad()
+@_no_grad
 def quantize_4bit(A: torch.Tensor, absmax: Optional[torch.Tensor] = None, out: Optional[torch.Tensor] = None,
                   blocksize: int = 64, compress_statistics: bool = False, quant_type: str = "nf4",
                   quant_storage: torch.dtype = torch.uint8, *, rounding: str = DEFAULT_ROUNDING):
@@ -163,7 +181,7 @@ def quantize_4bit(A: torch.Tensor, absmax: Optional[torch.Tensor] = None, out: O
     packed = torch.empty(((n + 1) // 2, 1), dtype=torch.uint8, device=dev)
     am = torch.empty(nblocks, dtype=torch.float32, device=dev)
     L = _lib.lib()
-    with torch.cuda.device(dev):
+    with _lib.device_guard(dev):
         rc = L.stm_nf4_quantize(src.data_ptr(), tag, n, blocksize, ROUNDING_RULES[rounding], packed.data_ptr(),
                                 am.data_ptr(), _lib.stream_handle(dev))
     _lib.check(rc, "stm_nf4_quantize")
@@ -181,7 +199,7 @@ def quantize_4bit(A: torch.Tensor, absmax: Optional[torch.Tensor] = None, out: O
     return packed, state
 
 
-@torch.no_grad()
+@_no_grad
 def dequantize_4bit(A: torch.Tensor, quant_state: Optional[QuantState] = None, absmax: Optional[torch.Tensor] = None,
                     out: Optional[torch.Tensor] = None, blocksize: int = 64, quant_type: str = "nf4",
                     *, dtype: Optional[torch.dtype] = None, shape: Optional[Sequence[int]] = None) -> torch.Tensor:
@@ -217,7 +235,7 @@ def dequantize_4bit(A: torch.Tensor, quant_state: Optional[QuantState] = None, a
     elif not out.is_contiguous() or out.numel() != n or out.dtype != dtype or out.device != dev:
         raise ValueError("out must be a contiguous tensor of the quant_state shape and dtype, on the packed "
                          "tensor's device")
-    with torch.cuda.device(dev):
+    with _lib.device_guard(dev):
         rc = _lib.lib().stm_nf4_dequantize(q.data_ptr(), am.data_ptr(), n, blocksize, out.data_ptr(),
                                            _lib.dtype_tag(dtype), _lib.stream_handle(dev))
     _lib.check(rc, "stm_nf4_dequantize")
@@ -230,7 +248,7 @@ def _ptr_array(values, ctype=None):
     return (ctype * max(1, len(values)))(*values)
 
 
-@torch.no_grad()
+@_no_grad
 def quantize_4bit_many(tensors: Sequence[torch.Tensor], blocksize: int = 64, *,
                        rounding: str = DEFAULT_ROUNDING) -> list:
     """``[quantize_4bit(t, blocksize=blocksize, rounding=rounding) for t in tensors]``
@@ -255,7 +273,7 @@ def quantize_4bit_many(tensors: Sequence[torch.Tensor], blocksize: int = 64, *,
     packed = [torch.empty(((n + 1) // 2, 1), dtype=torch.uint8, device=dev) for n in ns]
     ams = [torch.empty(-(-n // blocksize), dtype=torch.float32, device=dev) for n in ns]
     import ctypes
-    with torch.cuda.device(dev):
+    with _lib.device_guard(dev):
         rc = _lib.lib().stm_nf4_quantize_many(
             len(srcs), _ptr_array([x.data_ptr() for x in srcs]), _ptr_array(ns, ctypes.c_int64), tag, blocksize,
             ROUNDING_RULES[rounding], _ptr_array([p.data_ptr() for p in packed]),
@@ -270,7 +288,7 @@ def quantize_4bit_many(tensors: Sequence[torch.Tensor], blocksize: int = 64, *,
     return out
 
 
-@torch.no_grad()
+@_no_grad
 def dequantize_4bit_many(items: Sequence[tuple], *, dtype: Optional[torch.dtype] = None,
                          out: Optional[Sequence[torch.Tensor]] = None) -> list:
     """``[dequantize_4bit(packed, state, dtype=dtype) for packed, state in items]``
@@ -312,7 +330,7 @@ def dequantize_4bit_many(items: Sequence[tuple], *, dtype: Optional[torch.dtype]
                                           for o, n in zip(outs, ns)):
             raise ValueError("out must hold one contiguous tensor of each item's shape and the output dtype")
     import ctypes
-    with torch.cuda.device(dev):
+    with _lib.device_guard(dev):
         rc = _lib.lib().stm_nf4_dequantize_many(
             len(items), _ptr_array([q.data_ptr() for q in qs]), _ptr_array([a.data_ptr() for a in ams]),
             _ptr_array(ns, ctypes.c_int64), blocksize, _ptr_array([o.data_ptr() for o in outs]),
@@ -321,7 +339,7 @@ def dequantize_4bit_many(items: Sequence[tuple], *, dtype: Optional[torch.dtype]
     return outs
 
 
-@torch.no_grad()
+@_no_grad
 def dequantize_4bit_host(items: Sequence[tuple], device: torch.device) -> Optional[list]:
     """:func:`dequantize_4bit_many` for payloads in pinned host memory: the kernel
     reads the packed codes and absmax over the host link, so nothing is copied to
@@ -345,7 +363,7 @@ def dequantize_4bit_host(items: Sequence[tuple], device: torch.device) -> Option
             return None
         ns.append(n)
     outs = [torch.empty(tuple(st.shape), dtype=dtype, device=device) for st in states]
-    with torch.cuda.device(device):
+    with _lib.device_guard(device):
         rc = _lib.lib().stm_nf4_dequantize_host(
             len(items), _ptr_array([q.data_ptr() for q, _ in items]),
             _ptr_array([st.absmax.data_ptr() for st in states]), _ptr_array(ns, ctypes.c_int64), blocksize,
@@ -356,7 +374,7 @@ def dequantize_4bit_host(items: Sequence[tuple], device: torch.device) -> Option
     return outs
 
 
-@torch.no_grad()
+@_no_grad
 def stack_nf4(items: Sequence[tuple]) -> tuple:
     """One NF4 weight ``[sum N_i, K]`` from weights ``[N_i, K]`` that share K and
     the blocksize: ``(packed, QuantState)`` with the packed bytes and absmax of
@@ -421,7 +439,7 @@ def _check_weight(packed: torch.Tensor, absmax: torch.Tensor, N: int, K: int, bl
         raise ValueError(f"absmax holds {absmax.numel()} blocks, {-(-n // blocksize)} needed")
 
 
-@torch.no_grad()
+@_no_grad
 def nf4_gemm_fwd(x: torch.Tensor, packed: torch.Tensor, absmax: torch.Tensor, weight_shape: Sequence[int],
                  blocksize: int = 64, bias: Optional[torch.Tensor] = None, lora_t: Optional[torch.Tensor] = None,
                  lora_b: Optional[torch.Tensor] = None, out: Optional[torch.Tensor] = None) -> torch.Tensor:
@@ -438,7 +456,7 @@ def nf4_gemm_fwd(x: torch.Tensor, packed: torch.Tensor, absmax: torch.Tensor, we
         raise ValueError(f"x has {x.shape[-1]} features, weight expects {K}")
     tag = _gemm_dtype(x)
     lead = x.shape[:-1]
-    x2 = _aligned(x.reshape(-1, K))
+    x2 = _aligned(_rows(x, K))
     M = x2.shape[0]
     dev = x2.device
     _check_weight(packed, absmax, N, K, blocksize, dev)
@@ -455,7 +473,7 @@ def nf4_gemm_fwd(x: torch.Tensor, packed: torch.Tensor, absmax: torch.Tensor, we
         R = t.shape[1]
         if lb.shape != (N, R):
             raise ValueError(f"lora_b shape {tuple(lb.shape)} != ({N}, {R})")
-    with torch.cuda.device(dev):
+    with _lib.device_guard(dev):
         ws = _gemm_workspace(M, N, K, False, dev)
         rc = _lib.lib().stm_nf4_gemm_fwd(
             x2.data_ptr(), _aligned(packed).data_ptr(), _aligned(absmax, 4).data_ptr(),
@@ -464,10 +482,10 @@ def nf4_gemm_fwd(x: torch.Tensor, packed: torch.Tensor, absmax: torch.Tensor, we
             y.data_ptr(), M, N, K, blocksize, tag, ws.data_ptr() if ws is not None else None,
             4 * ws.numel() if ws is not None else 0, _lib.stream_handle(dev))
     _lib.check(rc, "stm_nf4_gemm_fwd")
-    return y.reshape(*lead, N)
+    return y if len(lead) == 1 else y.reshape(*lead, N)
 
 
-@torch.no_grad()
+@_no_grad
 def nf4_gemm_bwd_dx(dy: torch.Tensor, packed: torch.Tensor, absmax: torch.Tensor, weight_shape: Sequence[int],
                     blocksize: int = 64, lora_u: Optional[torch.Tensor] = None,
                     lora_at: Optional[torch.Tensor] = None, out: Optional[torch.Tensor] = None) -> torch.Tensor:
@@ -478,7 +496,7 @@ def nf4_gemm_bwd_dx(dy: torch.Tensor, packed: torch.Tensor, absmax: torch.Tensor
         raise ValueError(f"dy has {dy.shape[-1]} features, weight has {N} rows")
     tag = _gemm_dtype(dy)
     lead = dy.shape[:-1]
-    d2 = _aligned(dy.reshape(-1, N))
+    d2 = _aligned(_rows(dy, N))
     M = d2.shape[0]
     dev = d2.device
     _check_weight(packed, absmax, N, K, blocksize, dev)
@@ -492,7 +510,7 @@ def nf4_gemm_bwd_dx(dy: torch.Tensor, packed: torch.Tensor, absmax: torch.Tensor
         R = u.shape[1]
         if at.shape != (K, R):
             raise ValueError(f"lora_at shape {tuple(at.shape)} != ({K}, {R})")
-    with torch.cuda.device(dev):
+    with _lib.device_guard(dev):
         ws = _gemm_workspace(M, N, K, True, dev)
         rc = _lib.lib().stm_nf4_gemm_bwd_dx(
             d2.data_ptr(), _aligned(packed).data_ptr(), _aligned(absmax, 4).data_ptr(),
@@ -500,7 +518,7 @@ def nf4_gemm_bwd_dx(dy: torch.Tensor, packed: torch.Tensor, absmax: torch.Tensor
             dx.data_ptr(), M, N, K, blocksize, tag, ws.data_ptr() if ws is not None else None,
             4 * ws.numel() if ws is not None else 0, _lib.stream_handle(dev))
     _lib.check(rc, "stm_nf4_gemm_bwd_dx")
-    return dx.reshape(*lead, K)
+    return dx if len(lead) == 1 else dx.reshape(*lead, K)
 
 
 _OFFSETS_CACHE: "OrderedDict[tuple, tuple]" = OrderedDict()
@@ -529,7 +547,7 @@ def _device_offsets(host_off, dev: torch.device):
         return staged, off
     staged = torch.empty(host_off.shape[0], dtype=torch.int32, pin_memory=True)
     staged.numpy()[:] = host_off
-    with torch.cuda.device(dev):
+    with _lib.device_guard(dev):
         off = staged.to(dev, non_blocking=True)
         done = torch.cuda.Event()
         done.record(stream)
@@ -539,7 +557,7 @@ def _device_offsets(host_off, dev: torch.device):
     return staged, off
 
 
-@torch.no_grad()
+@_no_grad
 def nf4_grouped_gemm(x: torch.Tensor, packed: torch.Tensor, absmax: torch.Tensor, offsets: torch.Tensor,
                      expert_shape: Sequence[int], blocksize: int = 64, max_rows: Optional[int] = None,
                      backward: bool = False, out: Optional[torch.Tensor] = None) -> torch.Tensor:
@@ -594,13 +612,13 @@ def nf4_grouped_gemm(x: torch.Tensor, packed: torch.Tensor, absmax: torch.Tensor
     # the host copy of the offsets: validated by the library, and the forward's tile height
     lead = (xin.data_ptr(), _aligned(packed).data_ptr(), _aligned(absmax, 4).data_ptr(), off.data_ptr(),
             staged.data_ptr())
-    with torch.cuda.device(dev):
+    with _lib.device_guard(dev):
         rc = fn(*lead, E, int(max_rows), y.data_ptr(), N, K, blocksize, tag, _lib.stream_handle(dev))
     _lib.check(rc, "stm_nf4_grouped_gemm_" + ("bwd_dx" if backward else "fwd"))
     return y
 
 
-@torch.no_grad()
+@_no_grad
 def swiglu_fwd(gate_up: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """``silu(gate) * up`` of a stacked projection output ``gate_up`` [..., 2 I] = [gate | up].
 
@@ -612,18 +630,18 @@ def swiglu_fwd(gate_up: torch.Tensor, out: Optional[torch.Tensor] = None) -> tor
     if two_i % 2:
         raise ValueError("gate_up must have an even last dimension [gate | up]")
     inter = two_i // 2
-    gu = gate_up.reshape(-1, two_i).contiguous()
+    gu = _rows(gate_up, two_i).contiguous()
     rows = gu.shape[0]
     dev = gu.device
     h = _out_buffer(out, (rows, inter), gate_up.dtype, dev) if out is not None else \
         torch.empty((rows, inter), dtype=gate_up.dtype, device=dev)
-    with torch.cuda.device(dev):
+    with _lib.device_guard(dev):
         rc = _lib.lib().stm_swiglu_fwd(gu.data_ptr(), h.data_ptr(), rows, inter, tag, _lib.stream_handle(dev))
     _lib.check(rc, "stm_swiglu_fwd")
-    return h.reshape(*gate_up.shape[:-1], inter)
+    return h if gate_up.dim() == 2 else h.reshape(*gate_up.shape[:-1], inter)
 
 
-@torch.no_grad()
+@_no_grad
 def swiglu_bwd(grad_out: torch.Tensor, gate_up: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """Gradient of :func:`swiglu_fwd` with respect to ``gate_up``: [..., 2 I] = [d gate | d up]."""
     tag = _gemm_dtype(gate_up)
@@ -631,8 +649,8 @@ def swiglu_bwd(grad_out: torch.Tensor, gate_up: torch.Tensor, out: Optional[torc
     inter = two_i // 2
     if grad_out.shape[-1] != inter or grad_out.dtype != gate_up.dtype:
         raise ValueError("grad_out must be [..., I] in gate_up's dtype")
-    gu = gate_up.reshape(-1, two_i).contiguous()
-    dh = grad_out.reshape(-1, inter).contiguous()
+    gu = _rows(gate_up, two_i).contiguous()
+    dh = _rows(grad_out, inter).contiguous()
     rows = gu.shape[0]
     if dh.shape[0] != rows:
         raise ValueError("grad_out and gate_up have different row counts")
@@ -640,11 +658,11 @@ def swiglu_bwd(grad_out: torch.Tensor, gate_up: torch.Tensor, out: Optional[torc
     _on_device(dev, grad_out=dh)
     dgu = _out_buffer(out, (rows, two_i), gate_up.dtype, dev) if out is not None else \
         torch.empty((rows, two_i), dtype=gate_up.dtype, device=dev)
-    with torch.cuda.device(dev):
+    with _lib.device_guard(dev):
         rc = _lib.lib().stm_swiglu_bwd(dh.data_ptr(), gu.data_ptr(), dgu.data_ptr(), rows, inter, tag,
                                        _lib.stream_handle(dev))
     _lib.check(rc, "stm_swiglu_bwd")
-    return dgu.reshape(*gate_up.shape[:-1], two_i)
+    return dgu if gate_up.dim() == 2 else dgu.reshape(*gate_up.shape[:-1], two_i)
 
 
 # ------------------------------------------------------------ LoRA side products
@@ -671,7 +689,7 @@ def _ptr(t: Optional[torch.Tensor]):
     return t.data_ptr() if t is not None and t.numel() else None
 
 
-@torch.no_grad()
+@_no_grad
 def lora_down(x: torch.Tensor, lora_a: torch.Tensor, scaling: float = 1.0) -> torch.Tensor:
     """``scaling * x @ lora_a.T`` as [rows, R] in x's dtype (the ``T`` the fused
     forward takes as ``lora_t``); one pass over x, fp32 accumulation, one rounding."""
@@ -688,7 +706,7 @@ def lora_down(x: torch.Tensor, lora_a: torch.Tensor, scaling: float = 1.0) -> to
     _on_device(dev, lora_a=lora_a)
     a = _aligned(lora_a.to(x.dtype))
     t = torch.empty((M, R), dtype=x.dtype, device=dev)
-    with torch.cuda.device(dev):
+    with _lib.device_guard(dev):
         ws = _lora_workspace(M, K, R, 0, dev)
         rc = _lib.lib().stm_lora_down(_ptr(x2), _ptr(a), _ptr(t), M, K, R, float(scaling), tag, _ptr(ws),
                                       4 * ws.numel() if ws is not None else 0, _lib.stream_handle(dev))
@@ -696,7 +714,7 @@ def lora_down(x: torch.Tensor, lora_a: torch.Tensor, scaling: float = 1.0) -> to
     return t
 
 
-@torch.no_grad()
+@_no_grad
 def lora_dy(dy: torch.Tensor, lora_b: torch.Tensor, t: Optional[torch.Tensor] = None, scaling: float = 1.0):
     """``(scaling * dy @ lora_b, dy.T @ t)`` -- the rank-R input of the LoRA term of
     dX and the gradient of ``lora_b`` -- from one pass over dy. The second is None
@@ -706,7 +724,7 @@ def lora_dy(dy: torch.Tensor, lora_b: torch.Tensor, t: Optional[torch.Tensor] = 
     tag = _gemm_dtype(dy)
     if tuple(lora_b.shape) != (N, R):
         raise ValueError(f"lora_b shape {tuple(lora_b.shape)} != ({N}, {R})")
-    d2 = _aligned(dy.reshape(-1, N))
+    d2 = _aligned(_rows(dy, N))
     M = d2.shape[0]
     dev = d2.device
     _on_device(dev, lora_b=lora_b, t=t)
@@ -716,7 +734,7 @@ def lora_dy(dy: torch.Tensor, lora_b: torch.Tensor, t: Optional[torch.Tensor] = 
         t2 = _aligned(t.reshape(M, R).to(dy.dtype))
     u = torch.empty((M, R), dtype=dy.dtype, device=dev)
     db = torch.empty((N, R), dtype=dy.dtype, device=dev) if t is not None else None
-    with torch.cuda.device(dev):
+    with _lib.device_guard(dev):
         ws = _lora_workspace(M, N, R, 1, dev)
         rc = _lib.lib().stm_lora_dy(_ptr(d2), _ptr(b), _ptr(t2), _ptr(u), _ptr(db), M, N, R, float(scaling), tag,
                                     _ptr(ws), 4 * ws.numel() if ws is not None else 0, _lib.stream_handle(dev))
@@ -724,11 +742,11 @@ def lora_dy(dy: torch.Tensor, lora_b: torch.Tensor, t: Optional[torch.Tensor] = 
     return u, db
 
 
-@torch.no_grad()
+@_no_grad
 def lora_da(u: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
     """``u.T @ x`` ([R, K], x's dtype): the gradient of ``lora_a``; one pass over x."""
     K = x.shape[-1]
-    x2 = _aligned(x.reshape(-1, K))
+    x2 = _aligned(_rows(x, K))
     M = x2.shape[0]
     R = int(u.shape[-1])
     tag = _gemm_dtype(x)
@@ -736,7 +754,7 @@ def lora_da(u: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
     _on_device(dev, u=u)
     u2 = _aligned(u.reshape(M, R).to(x.dtype))
     da = torch.empty((R, K), dtype=x.dtype, device=dev)
-    with torch.cuda.device(dev):
+    with _lib.device_guard(dev):
         ws = _lora_workspace(M, K, R, 2, dev)
         rc = _lib.lib().stm_lora_da(_ptr(u2), _ptr(x2), _ptr(da), M, K, R, tag, _ptr(ws),
                                     4 * ws.numel() if ws is not None else 0, _lib.stream_handle(dev))

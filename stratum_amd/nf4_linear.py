@@ -112,7 +112,7 @@ class _NF4LinearFn(torch.autograd.Function):
     def backward(ctx, dy):
         x, packed, absmax, lora_a, lora_b, t = ctx.saved_tensors
         N, K = ctx.shape
-        dy2 = dy.reshape(-1, N).contiguous()
+        dy2 = (dy if dy.dim() == 2 else dy.reshape(-1, N)).contiguous()
         u = d_b = None
         if lora_a is not None:
             if lora_supported(lora_a.shape[0], N, dy2.shape[0]):
@@ -136,11 +136,11 @@ class _NF4LinearFn(torch.autograd.Function):
                 else:
                     dx = dy2 @ w
                 del w
-            dx = dx.reshape(*dy.shape[:-1], K)
+            dx = dx if dy.dim() == 2 else dx.reshape(*dy.shape[:-1], K)
         d_bias = dy2.sum(0).to(dy.dtype) if ctx.has_bias_grad else None
         d_a = None
         if lora_a is not None:
-            x2 = x.reshape(-1, K)
+            x2 = x if x.dim() == 2 else x.reshape(-1, K)
             if ctx.needs_input_grad[6]:
                 d_a = lora_da(u, x2) if lora_supported(lora_a.shape[0], K, x2.shape[0]) else u.t() @ x2  # [R, K]
                 d_a = d_a.to(lora_a.dtype)
@@ -159,8 +159,7 @@ def nf4_linear(x: torch.Tensor, quantized: torch.Tensor, quant_state: QuantState
     ``w_dense``: an already dequantized W (same dtype as x) that the library
     path uses instead of dequantizing (``NF4Linear.dense_weight``); the fused
     path ignores it. ``keep_weight_for_backward``: see the module docstring."""
-    shape = tuple(int(s) for s in quant_state.shape)
-    N, K = shape
+    shape = N, K = tuple(map(int, quant_state.shape))
     bs = quant_state.blocksize
     rank = lora_a.shape[0] if lora_a is not None else 0
     if x.is_cuda and x.dtype in (torch.bfloat16, torch.float16) and rank % 16 == 0:

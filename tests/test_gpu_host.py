@@ -319,3 +319,23 @@ def test_stream_load_and_quantize_from_checkpoint_bit_exact(cuda, tmp_path):
     m2 = M()
     stats2 = stream_load_and_quantize_module(m2, str(tmp_path), cache_dir=tmp_path / "cache")
     assert stats2.cache_hits == 1
+
+
+def test_operators_record_no_graph_and_follow_the_current_stream(cuda):
+    """With gradients on and inputs that require them, an operator's result has no
+    graph; the stream handle is the current stream's, as torch gives it."""
+    from stratum_amd import _lib
+    from stratum_amd.functional import (dequantize_4bit, lora_down, nf4_gemm_bwd_dx, nf4_gemm_fwd, quantize_4bit,
+                                        swiglu_fwd)
+    packed, st = quantize_4bit(seeded((128, 64), 1, 0.02, torch.float16).to(cuda))
+    x = seeded((3, 64), 2, 1.0, torch.bfloat16).to(cuda).requires_grad_(True)
+    dy = seeded((2, 3, 128), 3, 1.0, torch.bfloat16).to(cuda).requires_grad_(True)
+    a = seeded((16, 64), 4, 1.0, torch.bfloat16).to(cuda).requires_grad_(True)
+    outs = [nf4_gemm_fwd(x, packed, st.absmax, (128, 64)), nf4_gemm_bwd_dx(dy, packed, st.absmax, (128, 64)),
+            lora_down(x, a), swiglu_fwd(x), dequantize_4bit(packed, st)]
+    assert [tuple(o.shape) for o in outs] == [(3, 128), (2, 3, 64), (3, 16), (3, 32), (128, 64)]
+    assert torch.is_grad_enabled() and not any(o.requires_grad for o in outs)
+    for stream in (torch.cuda.default_stream(cuda), torch.cuda.Stream()):
+        with torch.cuda.stream(stream):
+            assert _lib.stream_handle(cuda) == torch.cuda.current_stream(cuda).cuda_stream == stream.cuda_stream
+            assert _lib.stream_handle(torch.device("cuda")) == stream.cuda_stream
