@@ -290,6 +290,16 @@ int stm_lora_da(const void* U, const void* X, void* dA, int64_t M, int64_t K, in
                 int64_t workspace_bytes, void* stream);
 
 /*
+ * The rank-R term by itself, for a base product that accumulates into it:
+ *   stm_lora_up: Y[M, C] = (bias[C] +) T[M, R] . L[C, R]^T     (transposed = 0, L = B)
+ *                Y[M, C] = (bias[C] +) T[M, R] . L[R, C]       (transposed = 1, L = A)
+ * fp32 accumulation, one rounding. bias may be NULL; R, sizes, alignment and dtype as
+ * above (C the column count); bias 2-byte aligned. Asynchronous on `stream`.
+ */
+int stm_lora_up(const void* T, const void* L, const void* bias, void* Y, int64_t M, int64_t C, int rank,
+                int transposed, int dtype, void* stream);
+
+/*
  * Host-only introspection used by the CPU test suite (no GPU work):
  * the 15 fp32 decision boundaries of a rounding rule (code > i iff s >= b[i]),
  * and the 65-cell table the quantize kernel indexes with

@@ -434,6 +434,105 @@ void launch_down_rows(const void* X, const void* A, void* T, int64_t M, int64_t 
     }
 }
 
+// Y[m, c] = (bias[c] +) sum_r T[m, r] L[c, r]: the rank-R term of the output (L = B) or,
+// with LT (L row-major [R, cols], L = A), of the input gradient, written once for the base
+// product to accumulate into. Bound by the write of Y. A wave holds the L fragments and the
+// bias of 64 columns in registers and walks 16-row groups of T; one v_mfma_f32_16x16x32
+// covers any rank up to 32 (ranks >= R load as zeros).
+//
+// MFMA row i of fragment f is column 32 (f / 2) + 8 (i / 4) + 4 (f % 2) + i % 4, so lane
+// (lr, lh) ends with two 16-byte chunks of row lr: lh and lh + 4 of the row's 128 bytes.
+// Lanes 8 apart trade one chunk each, and every store instruction then writes 8 whole
+// 128-byte lines. W [14336, 4096] at 8192 rows (235 MB): 40 us (5.9 TB/s)
+// against 72 for a plain library product; LT, [8192, 4096]: 16.7 against 25.7.
+template <typename Tr, bool LT>
+__global__ __launch_bounds__(256) void k_lora_up(const uint16_t* __restrict__ T, const uint16_t* __restrict__ L,
+                                                 const uint16_t* __restrict__ bias, uint16_t* __restrict__ Y,
+                                                 int64_t rows, int64_t cols, int R, int rows_per_block) {
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lr = lane & 15, lh = lane >> 4;
+    const int64_t c0 = ((int64_t)blockIdx.x * 4 + wave) * 64;
+    if (c0 >= cols) return;
+    const bool rank_in = 8 * lh < R;
+    uint4 w[4];
+    float b[4][4];
+#pragma unroll
+    for (int f = 0; f < 4; ++f) {
+        const int64_t col = c0 + 32 * (f >> 1) + 8 * (lr >> 2) + 4 * (f & 1) + (lr & 3);
+        w[f] = make_uint4(0, 0, 0, 0);
+        if (rank_in && col < cols) {
+            if constexpr (LT) {
+                uint32_t v[8];
+#pragma unroll
+                for (int r = 0; r < 8; ++r) v[r] = L[(int64_t)(8 * lh + r) * cols + col];
+                w[f] = make_uint4(v[0] | v[1] << 16, v[2] | v[3] << 16, v[4] | v[5] << 16, v[6] | v[7] << 16);
+            } else {
+                w[f] = *reinterpret_cast<const uint4*>(L + col * R + 8 * lh);
+            }
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int64_t bc = c0 + 32 * (f >> 1) + 8 * lh + 4 * (f & 1) + e;
+            b[f][e] = bias != nullptr && bc < cols ? Tr::to_f32(bias[bc]) : 0.f;
+        }
+    }
+    const int64_t m_begin = (int64_t)blockIdx.y * rows_per_block;
+    const int64_t m_end = m_begin + rows_per_block < rows ? m_begin + rows_per_block : rows;
+    const bool low = lr < 8;
+    // after the trade: chunk 0 goes to row lr % 8, chunk 1 to row lr % 8 + 8, both at column chunk
+    const int64_t col = c0 + 8 * (low ? lh : lh + 4);
+    const bool col_in = col < cols;
+    auto load = [&](int64_t m0) {
+        uint4 t = make_uint4(0, 0, 0, 0);
+        if (rank_in && m0 + lr < m_end) t = *reinterpret_cast<const uint4*>(T + (m0 + lr) * R + 8 * lh);
+        return t;
+    };
+    uint4 next = load(m_begin);
+    for (int64_t m0 = m_begin; m0 < m_end; m0 += 16) {
+        const uint4 t = next;
+        next = load(m0 + 16);
+        uint32_t q[2][4];
+#pragma unroll
+        for (int f = 0; f < 4; ++f) {
+            const f32x4_t init = {b[f][0], b[f][1], b[f][2], b[f][3]};
+            const f32x4_t d = mfma16x32<Tr>(w[f], t, init);
+            q[f >> 1][2 * (f & 1)] = Tr::pack2(d[0], d[1]);
+            q[f >> 1][2 * (f & 1) + 1] = Tr::pack2(d[2], d[3]);
+        }
+        uint32_t o0[4], o1[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const uint32_t give = low ? q[1][e] : q[0][e];
+            // row_ror:8: lane lr of a 16-lane row receives from lane lr ^ 8
+            const uint32_t got = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)give, 0x128, 0xf, 0xf, false);
+            o0[e] = low ? q[0][e] : got;
+            o1[e] = low ? got : q[1][e];
+        }
+        const int64_t m = m0 + (lr & 7);
+        if (col_in && m < m_end)
+            *reinterpret_cast<uint4*>(Y + m * cols + col) = make_uint4(o0[0], o0[1], o0[2], o0[3]);
+        if (col_in && m + 8 < m_end)
+            *reinterpret_cast<uint4*>(Y + (m + 8) * cols + col) = make_uint4(o1[0], o1[1], o1[2], o1[3]);
+    }
+}
+
+template <typename Tr>
+void launch_up(const void* T, const void* L, const void* bias, void* Y, int64_t M, int64_t C, int R, bool lt,
+               hipStream_t st) {
+    const int64_t ncb = (C + 255) / 256;
+    // 128 rows per work-group, fewer while that leaves the GPU with under four work-groups per CU;
+    // rows grow past it only where the grid's second dimension ends (65535)
+    int64_t rpb = 128;
+    while (rpb > 16 && ncb * ((M + rpb - 1) / rpb) < 1024) rpb /= 2;
+    while ((M + rpb - 1) / rpb > 65535) rpb *= 2;
+    const dim3 grid((unsigned)ncb, (unsigned)((M + rpb - 1) / rpb)), block(256);
+    const auto *t = (const uint16_t*)T, *l = (const uint16_t*)L, *b = (const uint16_t*)bias;
+    if (lt)
+        hipLaunchKernelGGL((k_lora_up<Tr, true>), grid, block, 0, st, t, l, b, (uint16_t*)Y, M, C, R, (int)rpb);
+    else
+        hipLaunchKernelGGL((k_lora_up<Tr, false>), grid, block, 0, st, t, l, b, (uint16_t*)Y, M, C, R, (int)rpb);
+}
+
 int rank_padded(int R) { return R <= 16 ? 16 : 32; }
 
 // Blocks over the rows: about two work-groups per CU of MI355X's 256 in total,
@@ -642,4 +741,19 @@ extern "C" int stm_lora_da(const void* U, const void* X, void* dA, int64_t M, in
     launch_pass(a, dtype, false, true, dim3((unsigned)p.ncb, (unsigned)p.nrb), st);
     launch_reduce(part, (int)p.nrb, K, rank, 1.f, dA, true, dtype, st);
     return check_launch("lora_da");
+}
+
+extern "C" int stm_lora_up(const void* T, const void* L, const void* bias, void* Y, int64_t M, int64_t C, int rank,
+                           int transposed, int dtype, void* stream) {
+    int rc = check_common("lora_up", M, C, rank, dtype);
+    if (rc) return rc;
+    if (M == 0 || C == 0) return STM_OK;
+    if ((rc = check_ptrs("lora_up", {T, L, Y}))) return rc;
+    if (bias && !aligned(bias, 2)) return set_error(STM_ERR_INVALID, "lora_up: bias not 2-byte aligned");
+    hipStream_t st = (hipStream_t)stream;
+    if (dtype == STM_BF16)
+        launch_up<BF16>(T, L, bias, Y, M, C, rank, transposed != 0, st);
+    else
+        launch_up<F16>(T, L, bias, Y, M, C, rank, transposed != 0, st);
+    return check_launch("lora_up");
 }

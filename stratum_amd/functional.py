@@ -760,3 +760,29 @@ def lora_da(u: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
                                     4 * ws.numel() if ws is not None else 0, _lib.stream_handle(dev))
     _lib.check(rc, "stm_lora_da")
     return da
+
+
+@_no_grad
+def lora_up(t: torch.Tensor, lora: torch.Tensor, bias: Optional[torch.Tensor] = None,
+            transposed: bool = False) -> torch.Tensor:
+    """``t @ lora.T (+ bias)`` with lora [C, R], or ``t @ lora (+ bias)`` with lora [R, C]
+    when ``transposed``: the rank-R term as a tensor [rows, C] of t's dtype, for a base
+    product that accumulates into it; fp32 accumulation, one rounding."""
+    M, R = int(t.shape[0]), int(t.shape[1])
+    C = int(lora.shape[1 if transposed else 0])
+    tag = _gemm_dtype(t)
+    if tuple(lora.shape) != ((R, C) if transposed else (C, R)):
+        raise ValueError(f"lora shape {tuple(lora.shape)} does not match rank {R}")
+    if bias is not None and tuple(bias.shape) != (C,):
+        raise ValueError(f"bias shape {tuple(bias.shape)} != ({C},)")
+    t2 = _aligned(t)
+    dev = t2.device
+    _on_device(dev, lora=lora, bias=bias)
+    lo = _aligned(lora.to(t.dtype))
+    b = bias.to(t.dtype).contiguous() if bias is not None else None
+    y = torch.empty((M, C), dtype=t.dtype, device=dev)
+    with _lib.device_guard(dev):
+        rc = _lib.lib().stm_lora_up(_ptr(t2), _ptr(lo), _ptr(b), _ptr(y), M, C, R, int(transposed), tag,
+                                    _lib.stream_handle(dev))
+    _lib.check(rc, "stm_lora_up")
+    return y

@@ -43,7 +43,7 @@ import torch.nn.functional as F
 import os
 
 from .functional import (QuantState, dequantize_4bit, fused_supported, lora_da, lora_down, lora_dy, lora_supported,
-                         nf4_gemm_bwd_dx, nf4_gemm_fwd)
+                         lora_up, nf4_gemm_bwd_dx, nf4_gemm_fwd)
 
 _DEFAULT_FUSED_MAX_ROWS = 768
 # With a LoRA adapter the fused kernels fold the rank-R terms into their
@@ -95,8 +95,11 @@ class _NF4LinearFn(torch.autograd.Function):
             if t is not None:
                 # rank-R term (and bias) first, then the base GEMM accumulates into it
                 # (beta = 1): no separate full-size add
-                lb_t = lora_b.to(x.dtype).t()
-                y2 = torch.addmm(b, t, lb_t) if b is not None else t @ lb_t
+                if lora_supported(lora_b.shape[1], w.shape[0], t.shape[0]):
+                    y2 = lora_up(t, lora_b, b)
+                else:
+                    lb_t = lora_b.to(x.dtype).t()
+                    y2 = torch.addmm(b, t, lb_t) if b is not None else t @ lb_t
                 y = y2.addmm_(x.reshape(-1, x.shape[-1]), w.t()).reshape(*x.shape[:-1], w.shape[0])
             else:
                 y = F.linear(x, w, b)
@@ -132,7 +135,9 @@ class _NF4LinearFn(torch.autograd.Function):
                     dequantize_4bit(packed, absmax=absmax, blocksize=ctx.blocksize, dtype=dy2.dtype, shape=ctx.shape)
                 ctx.w = None
                 if u is not None:
-                    dx = (u @ lora_a.to(dy2.dtype)).addmm_(dy2, w)     # rank-R term, then the base GEMM into it
+                    # rank-R term, then the base GEMM into it
+                    dx = (lora_up(u, lora_a, transposed=True) if lora_supported(u.shape[1], K, u.shape[0])
+                          else u @ lora_a.to(dy2.dtype)).addmm_(dy2, w)
                 else:
                     dx = dy2 @ w
                 del w

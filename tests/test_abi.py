@@ -236,6 +236,11 @@ def test_lora_arguments_are_rejected_without_a_gpu(L):
     assert L.stm_lora_down(p + 2, p, p, 64, 256, 16, 1.0, 1, p, ws_need, None) == -1
     assert L.stm_lora_dy(p, None, p, p, p, 64, 256, 16, 1.0, 1, p, 1 << 30, None) == -1
     assert L.stm_lora_da(p, p, None, 64, 256, 16, 1, p, 1 << 30, None) == -1
+    assert L.stm_lora_up(p, p, None, p, 64, 256, 12, 0, 1, None) == -2
+    assert L.stm_lora_up(p, p, None, p, 64, 250, 16, 0, 1, None) == -2
+    assert L.stm_lora_up(p, p + 2, None, p, 64, 256, 16, 1, 1, None) == -1
+    assert L.stm_lora_up(p, p, p + 1, p, 64, 256, 16, 0, 1, None) == -1
+    assert L.stm_lora_up(p, p, None, p, 0, 256, 16, 0, 1, None) == 0
     # workspace too small or missing
     assert L.stm_lora_down(p, p, p, 64, 256, 16, 1.0, 1, p, ws_need - 16, None) == -1
     assert "workspace" in _err(L)

@@ -145,3 +145,27 @@ def test_lora_entry_points_replay_correctly_in_a_hip_graph(cuda):
         assert torch.equal(u_g, u_e) and torch.equal(db_g, db_e), i
         assert torch.equal(da_g, da_e), i
         del junk
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M,C,R", SHAPES + [(17, 64, 32), (33, 72, 16), (8192, 256, 16)])
+def test_lora_up(cuda, dtype, M, C, R):
+    """t @ lora^T (+ bias) in both layouts of lora: one rounding of an fp32 sum of at most 33
+    products, so each value is within one unit in the last place of the result (2^-8 / 2^-11
+    of it) plus the sum's own error, 34 * 2^-24 of the sum of magnitudes."""
+    from stratum_amd.functional import lora_up
+    t = seeded((M, R), 8, 1.0, dtype, cuda)
+    b = seeded((C, R), 9, 0.05, dtype, cuda)
+    bias = seeded((C,), 10, 0.1, dtype, cuda)
+    for with_bias in (None, bias):
+        exact = t.double() @ b.double().t().contiguous()
+        scale = t.double().abs() @ b.double().abs().t().contiguous()
+        if with_bias is not None:
+            exact, scale = exact + bias.double(), scale + bias.double().abs()
+        unit = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
+        tiny = 0.0 if dtype == torch.bfloat16 else 2.0 ** -25  # half the spacing of fp16's subnormals
+        limit = unit * exact.abs() + 34 * 2.0 ** -24 * scale + tiny
+        for lora, transposed in ((b, False), (b.t().contiguous(), True)):
+            y = lora_up(t, lora, with_bias, transposed=transposed)
+            assert y.shape == (M, C) and y.dtype == dtype
+            assert bool(((y.double() - exact).abs() <= limit).all())
