@@ -300,6 +300,20 @@ int stm_lora_up(const void* T, const void* L, const void* bias, void* Y, int64_t
                 int transposed, int dtype, void* stream);
 
 /*
+ * Operands of one product that computes the base projection and the LoRA term together,
+ * Y = [X | T | 0] . [W | L | 0]^T over K + 64 columns (the term then shares the base's
+ * fp32 sums and its one rounding):
+ *   stm_lora_down_aug:      T as stm_lora_down (its workspace too) and XA[M, K + 64] = [X | T | 0]
+ *   stm_nf4_dequantize_aug: out[N, K + 64] = [W | L | 0], W the dequantized weight, L [N, lora_rank]
+ * K a multiple of 8 (aug: 64), M (K + 64) below 2^30; dtype STM_BF16 or STM_F16; packed 4-byte,
+ * the 16-bit operands 16-byte aligned. Asynchronous on `stream`.
+ */
+int stm_lora_down_aug(const void* X, const void* A, void* T, void* XA, int64_t M, int64_t K, int rank, float scaling,
+                      int dtype, void* workspace, int64_t workspace_bytes, void* stream);
+int stm_nf4_dequantize_aug(const uint8_t* packed, const float* absmax, const void* L, int lora_rank, void* out,
+                           int64_t N, int64_t K, int blocksize, int dtype, void* stream);
+
+/*
  * Host-only introspection used by the CPU test suite (no GPU work):
  * the 15 fp32 decision boundaries of a rounding rule (code > i iff s >= b[i]),
  * and the 65-cell table the quantize kernel indexes with

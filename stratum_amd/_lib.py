@@ -54,6 +54,8 @@ SIGNATURES = {
     "stm_lora_workspace_bytes": ([_I64, _I64, _I, _I], _I64),
     "stm_lora_down": ([_P, _P, _P, _I64, _I64, _I, ctypes.c_float, _I, _P, _I64, _P], _I),
     "stm_lora_dy": ([_P, _P, _P, _P, _P, _I64, _I64, _I, ctypes.c_float, _I, _P, _I64, _P], _I),
+    "stm_lora_down_aug": ([_P, _P, _P, _P, _I64, _I64, _I, ctypes.c_float, _I, _P, _I64, _P], _I),
+    "stm_nf4_dequantize_aug": ([_P, _P, _P, _I, _P, _I64, _I64, _I, _I, _P], _I),
     "stm_lora_up": ([_P, _P, _P, _P, _I64, _I64, _I, _I, _I, _P], _I),
     "stm_lora_da": ([_P, _P, _P, _I64, _I64, _I, _I, _P, _I64, _P], _I),
     "stm_nf4_decision_boundaries": ([_I, _P], _I),

@@ -204,6 +204,26 @@ int stm_nf4_dequantize(const uint8_t* packed, const float* absmax, int64_t n, in
     return launch_dequantize(packed, absmax, n, blocksize, out, out_dtype, (hipStream_t)stream);
 }
 
+int stm_nf4_dequantize_aug(const uint8_t* packed, const float* absmax, const void* L, int lora_rank, void* out,
+                           int64_t N, int64_t K, int blocksize, int dtype, void* stream) {
+    g_err[0] = 0;
+    if (N < 0 || K < 0) return set_error(STM_ERR_INVALID, "dequantize_aug: negative size");
+    if (dtype != STM_BF16 && dtype != STM_F16)
+        return set_error(STM_ERR_INVALID, "dequantize_aug: dtype must be bf16 or fp16");
+    if (!valid_blocksize(blocksize))
+        return set_error(STM_ERR_INVALID, "dequantize_aug: blocksize %d not a power of two in [64, 4096]", blocksize);
+    if (lora_rank < 8 || lora_rank > 32 || lora_rank % 8)
+        return set_error(STM_ERR_UNSUPPORTED, "dequantize_aug: rank %d (needs 8, 16, 24 or 32)", lora_rank);
+    if (N == 0) return STM_OK;
+    // 32-bit word indices
+    if (K % 64 || K == 0 || N > 0x7FFFFFFFLL / (K / 8 + 8))
+        return set_error(STM_ERR_UNSUPPORTED, "dequantize_aug: [%lld, %lld]", (long long)N, (long long)K);
+    if (!packed || !absmax || !L || !out) return set_error(STM_ERR_INVALID, "dequantize_aug: NULL pointer");
+    if (!aligned(packed, 4) || !aligned(L, 16) || !aligned(out, 16))
+        return set_error(STM_ERR_INVALID, "dequantize_aug: operand not aligned");
+    return launch_dequantize_aug(packed, absmax, L, N, K, lora_rank, blocksize, out, dtype, (hipStream_t)stream);
+}
+
 int stm_nf4_quantize_many(int count, const void* const* A, const int64_t* n, int dtype, int blocksize, int rounding,
                           uint8_t* const* packed, float* const* absmax, void* stream) {
     g_err[0] = 0;

@@ -63,6 +63,9 @@ int grouped_tile_rows(const int32_t* offsets, int num_experts);
 
 int launch_quantize(const void* A, int dtype, int64_t n, int blocksize, const CellTable& tab, uint8_t* packed,
                     float* absmax, hipStream_t stream);
+// Rows of cols + 64 columns: the dequantized row, L's R ranks, zeros (16-bit types).
+int launch_dequantize_aug(const uint8_t* packed, const float* absmax, const void* L, int64_t rows, int64_t cols, int R,
+                          int bs, void* out, int dtype, hipStream_t stream);
 int launch_dequantize(const uint8_t* packed, const float* absmax, int64_t n, int blocksize, void* out, int out_dtype,
                       hipStream_t stream);
 // Many tensors of one dtype / blocksize (/ rule): batched launches of whole

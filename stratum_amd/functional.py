@@ -786,3 +786,55 @@ def lora_up(t: torch.Tensor, lora: torch.Tensor, bias: Optional[torch.Tensor] = 
                                     _lib.stream_handle(dev))
     _lib.check(rc, "stm_lora_up")
     return y
+
+
+LORA_AUG_PAD = 64
+
+
+def lora_aug_supported(rank: int, rows: int, N: int, K: int) -> bool:
+    """Shapes that :func:`lora_down_aug` and :func:`dequantize_4bit_aug` take."""
+    return (lora_supported(rank, K, rows) and K % 64 == 0 and rows * (K + LORA_AUG_PAD) < 1 << 30
+            and N * (K // 8 + 8) < 1 << 31)
+
+
+@_no_grad
+def lora_down_aug(x: torch.Tensor, lora_a: torch.Tensor, scaling: float = 1.0):
+    """``(t, [x | t | 0])`` for x [rows, K]: :func:`lora_down` and, from the same pass over x,
+    the left operand [rows, K + 64] of a product that adds the LoRA term itself."""
+    M, K = x.shape
+    R = int(lora_a.shape[0])
+    tag = _gemm_dtype(x)
+    if tuple(lora_a.shape) != (R, K):
+        raise ValueError(f"lora_a shape {tuple(lora_a.shape)} != ({R}, {K})")
+    x2 = _aligned(x)
+    dev = x2.device
+    _on_device(dev, lora_a=lora_a)
+    a = _aligned(lora_a.to(x.dtype))
+    t = torch.empty((M, R), dtype=x.dtype, device=dev)
+    xa = torch.empty((M, K + LORA_AUG_PAD), dtype=x.dtype, device=dev)
+    with _lib.device_guard(dev):
+        ws = _lora_workspace(M, K, R, 0, dev)
+        rc = _lib.lib().stm_lora_down_aug(_ptr(x2), _ptr(a), _ptr(t), _ptr(xa), M, K, R, float(scaling), tag, _ptr(ws),
+                                          4 * ws.numel() if ws is not None else 0, _lib.stream_handle(dev))
+    _lib.check(rc, "stm_lora_down_aug")
+    return t, xa
+
+
+@_no_grad
+def dequantize_4bit_aug(packed: torch.Tensor, absmax: torch.Tensor, weight_shape: Sequence[int], blocksize: int,
+                        lora_b: torch.Tensor, dtype: torch.dtype) -> torch.Tensor:
+    """``[W | lora_b | 0]`` ([N, K + 64]), the right operand to :func:`lora_down_aug`'s left one."""
+    N, K = int(weight_shape[0]), int(weight_shape[1])
+    dev = packed.device
+    _check_weight(packed, absmax, N, K, blocksize, dev)
+    _on_device(dev, lora_b=lora_b)
+    if lora_b.dim() != 2 or lora_b.shape[0] != N:
+        raise ValueError(f"lora_b shape {tuple(lora_b.shape)} does not match {N} rows")
+    b = _aligned(lora_b.to(dtype))
+    out = torch.empty((N, K + LORA_AUG_PAD), dtype=dtype, device=dev)
+    with _lib.device_guard(dev):
+        rc = _lib.lib().stm_nf4_dequantize_aug(_aligned(packed, 4).data_ptr(), _aligned(absmax, 4).data_ptr(), _ptr(b),
+                                               int(b.shape[1]), _ptr(out), N, K, blocksize, _lib.dtype_tag(dtype),
+                                               _lib.stream_handle(dev))
+    _lib.check(rc, "stm_nf4_dequantize_aug")
+    return out

@@ -42,8 +42,8 @@ import torch.nn.functional as F
 
 import os
 
-from .functional import (QuantState, dequantize_4bit, fused_supported, lora_da, lora_down, lora_dy, lora_supported,
-                         lora_up, nf4_gemm_bwd_dx, nf4_gemm_fwd)
+from .functional import (QuantState, dequantize_4bit, dequantize_4bit_aug, fused_supported, lora_aug_supported, lora_da,
+                         lora_down, lora_down_aug, lora_dy, lora_supported, lora_up, nf4_gemm_bwd_dx, nf4_gemm_fwd)
 
 _DEFAULT_FUSED_MAX_ROWS = 768
 # With a LoRA adapter the fused kernels fold the rank-R terms into their
@@ -71,15 +71,32 @@ def _mm_scaled(a: torch.Tensor, b: torch.Tensor, scaling: float) -> torch.Tensor
     return torch.addmm(a.new_empty(()), a, b, beta=0, alpha=scaling)  # beta = 0: the input is never read
 
 
+def _augment(x, packed, absmax, shape, lora_a, lora_b, w_dense) -> bool:
+    """Whether the library path's forward runs one product over K + 64 columns, [x | t] [W | B]^T.
+
+    It saves the rank-R term's write of Y and the base product's read of it (4 N bytes a row) for a
+    copy of x (2 K bytes a row) and 64 / K more products, so it is taken for N >= 2 K.
+    W [14336, 4096] at 8192 rows, us: product 656 -> 616, no 40 for the term, copy 15 -> 26,
+    dequantize 26 -> 31. At N = K the library product over K + 64 columns takes back what is
+    saved ([4096, 4096] at 4096 rows: 92 + 11 for product and term, 88 + 12 with the copy)."""
+    N, K = shape
+    rows = x.numel() // max(K, 1)
+    return (N >= 2 * K and rows > 64 and w_dense is None and packed.dtype == torch.uint8
+            and absmax.dtype == torch.float32 and packed.device == absmax.device == x.device
+            and lora_aug_supported(lora_a.shape[0], rows, N, K))
+
+
 class _NF4LinearFn(torch.autograd.Function):
     """y = x . W^T (+ bias) (+ scaling * (x . A^T) . B^T) with W frozen in NF4."""
 
     @staticmethod
     def forward(ctx, x, packed, absmax, shape, blocksize, bias, lora_a, lora_b, scaling, fused, w_dense=None,
                 keep_w=True):
-        t = None
+        t = xa = None
         if lora_a is not None:
-            if lora_supported(lora_a.shape[0], x.shape[-1], x.numel() // max(x.shape[-1], 1)):
+            if not fused and _augment(x, packed, absmax, shape, lora_a, lora_b, w_dense):
+                t, xa = lora_down_aug(x if x.dim() == 2 else x.reshape(-1, x.shape[-1]), lora_a, scaling)
+            elif lora_supported(lora_a.shape[0], x.shape[-1], x.numel() // max(x.shape[-1], 1)):
                 t = lora_down(x, lora_a, scaling)
             else:
                 t = _mm_scaled(x.reshape(-1, x.shape[-1]), lora_a.t().to(x.dtype), scaling)
@@ -87,12 +104,18 @@ class _NF4LinearFn(torch.autograd.Function):
             y = nf4_gemm_fwd(x, packed, absmax, shape, blocksize, bias=bias, lora_t=t,
                              lora_b=lora_b.to(x.dtype) if lora_b is not None else None)
         else:
-            if w_dense is not None and w_dense.dtype == x.dtype:
+            if xa is not None:
+                wa = dequantize_4bit_aug(packed, absmax, shape, blocksize, lora_b, x.dtype)
+                w = wa[:, :shape[1]]
+            elif w_dense is not None and w_dense.dtype == x.dtype:
                 w = w_dense
             else:
                 w = dequantize_4bit(packed, absmax=absmax, blocksize=blocksize, dtype=x.dtype, shape=shape)
             b = bias.to(x.dtype) if bias is not None else None
-            if t is not None:
+            if xa is not None:
+                y = F.linear(xa, wa, b)
+                y = y if x.dim() == 2 else y.reshape(*x.shape[:-1], w.shape[0])
+            elif t is not None:
                 # rank-R term (and bias) first, then the base GEMM accumulates into it
                 # (beta = 1): no separate full-size add
                 if lora_supported(lora_b.shape[1], w.shape[0], t.shape[0]):

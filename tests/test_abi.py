@@ -241,6 +241,14 @@ def test_lora_arguments_are_rejected_without_a_gpu(L):
     assert L.stm_lora_up(p, p + 2, None, p, 64, 256, 16, 1, 1, None) == -1
     assert L.stm_lora_up(p, p, p + 1, p, 64, 256, 16, 0, 1, None) == -1
     assert L.stm_lora_up(p, p, None, p, 0, 256, 16, 0, 1, None) == 0
+    assert L.stm_lora_down_aug(p, p, p, p, 64, 256, 12, 1.0, 1, p, ws_need, None) == -2
+    assert L.stm_lora_down_aug(p, p, p, p, 1 << 20, 1024, 16, 1.0, 1, p, 1 << 40, None) == -2  # past one buffer range
+    assert L.stm_lora_down_aug(p, p, p, p + 2, 64, 256, 16, 1.0, 1, p, ws_need, None) == -1
+    assert L.stm_lora_down_aug(p, p, p, p, 64, 256, 16, 1.0, 1, p, ws_need - 16, None) == -1
+    assert L.stm_nf4_dequantize_aug(p, p, p, 16, p, 64, 96, 64, 1, None) == -2
+    assert L.stm_nf4_dequantize_aug(p, p, p, 40, p, 64, 128, 64, 1, None) == -2
+    assert L.stm_nf4_dequantize_aug(p, p, p, 16, p, 64, 128, 64, 2, None) == -1
+    assert L.stm_nf4_dequantize_aug(p, p, p + 2, 16, p, 64, 128, 64, 1, None) == -1
     # workspace too small or missing
     assert L.stm_lora_down(p, p, p, 64, 256, 16, 1.0, 1, p, ws_need - 16, None) == -1
     assert "workspace" in _err(L)

@@ -169,3 +169,59 @@ def test_lora_up(cuda, dtype, M, C, R):
             y = lora_up(t, lora, with_bias, transposed=transposed)
             assert y.shape == (M, C) and y.dtype == dtype
             assert bool(((y.double() - exact).abs() <= limit).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M,K,R", [(1, 64, 8), (65, 320, 24), (700, 1024, 16), (130, 4096, 32), (2000, 576, 16)])
+def test_lora_down_aug(cuda, dtype, M, K, R):
+    """The augmented left operand: x, lora_down's t and zeros, bit for bit."""
+    from stratum_amd.functional import lora_down, lora_down_aug
+    x = seeded((M, K), 11, 1.0, dtype, cuda)
+    a = seeded((R, K), 12, 0.05, dtype, cuda)
+    t, xa = lora_down_aug(x, a, 2.0)
+    assert torch.equal(xa[:, :K], x) and torch.equal(xa[:, K:K + R], t) and not xa[:, K + R:].any()
+    if M > 64:  # up to 64 rows lora_down sums in another order
+        assert torch.equal(t, lora_down(x, a, 2.0))
+    else:
+        assert rel(t, 2.0 * (x.float() @ a.float().t().contiguous())) <= TOL[dtype]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("N,K,R,bs", [(1, 64, 8, 64), (33, 320, 24, 128), (3072, 1024, 16, 64), (9000, 4032, 32, 64)])
+def test_dequantize_aug(cuda, dtype, N, K, R, bs):
+    """The augmented right operand: dequantize_4bit's weight, lora_b and zeros, bit for bit."""
+    from stratum_amd.functional import dequantize_4bit, dequantize_4bit_aug, quantize_4bit
+    q, st = quantize_4bit(seeded((N, K), 13, 0.02, torch.float16, cuda), blocksize=bs)
+    b = seeded((N, R), 14, 0.05, dtype, cuda)
+    wa = dequantize_4bit_aug(q, st.absmax, (N, K), bs, b, dtype)
+    assert torch.equal(wa[:, :K], dequantize_4bit(q, st, dtype=dtype))
+    assert torch.equal(wa[:, K:K + R], b) and not wa[:, K + R:].any()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("keep", [True, False])
+@pytest.mark.parametrize("N,K,rows,bias", [(768, 384, (3, 41), True), (704, 320, (1100,), False), (640, 384, (130,), True)])
+def test_library_path_step_with_and_without_augmentation(cuda, dtype, keep, N, K, rows, bias, monkeypatch):
+    """A LoRA step on the library path at N = 2 K (one product over K + 64 columns), above it
+    and below it (the base product added to the rank-R term), 2-D and 3-D, against fp32."""
+    from stratum_amd.functional import dequantize_4bit, quantize_4bit
+    from stratum_amd.nf4_linear import NF4LoRALinear
+    monkeypatch.setenv("STRATUM_NF4_FUSED_MAX_ROWS", "0")
+    q, st = quantize_4bit(seeded((N, K), 15, 0.02, torch.float16, cuda))
+    bv = seeded((N,), 16, 0.1, dtype, cuda) if bias else None
+    lin = NF4LoRALinear(q, st, bv, r=16, lora_alpha=32.0, dtype=dtype)
+    lin.keep_weight_for_backward = keep
+    with torch.no_grad():
+        lin.lora_A.copy_(seeded((16, K), 17, 0.05, dtype, cuda))
+        lin.lora_B.copy_(seeded((N, 16), 18, 0.05, dtype, cuda))
+    x = seeded((*rows, K), 19, 1.0, dtype, cuda).requires_grad_(True)
+    dy = seeded((*rows, N), 20, 1.0, dtype, cuda)
+    y = lin(x)
+    y.backward(dy)
+    w = dequantize_4bit(q, st, dtype=dtype).float()
+    xf = x.detach().float().reshape(-1, K).requires_grad_(True)
+    a, b = (p.detach().float().requires_grad_(True) for p in (lin.lora_A, lin.lora_B))
+    ref = xf @ w.t() + 2.0 * (xf @ a.t()) @ b.t() + (bv.float() if bias else 0.0)
+    ref.backward(dy.float().reshape(-1, N))
+    for got, want in ((y, ref), (x.grad, xf.grad), (lin.lora_A.grad, a.grad), (lin.lora_B.grad, b.grad)):
+        assert rel(got.detach().reshape(want.shape), want.detach()) <= TOL[dtype]
