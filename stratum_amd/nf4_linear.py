@@ -82,6 +82,8 @@ def _augment(x, packed, absmax, shape, lora_a, lora_b, w_dense) -> bool:
     N, K = shape
     rows = x.numel() // max(K, 1)
     return (N >= 2 * K and rows > 64 and w_dense is None and packed.dtype == torch.uint8
+            # the padding would hide adapters that don't match; the other route refuses them
+            and tuple(lora_b.shape) == (N, lora_a.shape[0])
             and absmax.dtype == torch.float32 and packed.device == absmax.device == x.device
             and lora_aug_supported(lora_a.shape[0], rows, N, K))
 
