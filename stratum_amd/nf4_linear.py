@@ -120,7 +120,7 @@ class _NF4LinearFn(torch.autograd.Function):
             elif t is not None:
                 # rank-R term (and bias) first, then the base GEMM accumulates into it
                 # (beta = 1): no separate full-size add
-                if lora_supported(lora_b.shape[1], w.shape[0], t.shape[0]):
+                if lora_supported(lora_b.shape[1], w.shape[0], t.shape[0]) and (b is None or b.shape == w.shape[:1]):
                     y2 = lora_up(t, lora_b, b)
                 else:
                     lb_t = lora_b.to(x.dtype).t()

@@ -29,6 +29,12 @@ def operators(monkeypatch):
         t = scaling * x @ a.t()
         return t, torch.cat([x, pad(t, 64)], 1)
 
+    def up(t, lora, bias=None, transposed=False):
+        assert bias is None or tuple(bias.shape) == (lora.shape[1 if transposed else 0],)  # as the operator
+        y = t @ lora if transposed else t @ lora.t()
+        return y if bias is None else y + bias
+
+    put("lora_up", up)
     put("lora_down", lambda x, a, scaling=1.0: scaling * x.reshape(-1, x.shape[-1]) @ a.t())
     put("lora_down_aug", down_aug)
     put("dequantize_4bit", lambda packed, **kw: packed.weight.to(kw["dtype"]))
@@ -81,3 +87,13 @@ def test_adapters_of_one_rank_take_the_augmented_product(operators, rank):
     y = apply(packed, absmax, x, a, b)
     assert "lora_down_aug" in operators and "dequantize_4bit_aug" in operators
     assert close(y, reference(packed, x, a, b))
+
+
+@pytest.mark.parametrize("N,K", [(256, 128), (128, 128)])
+@pytest.mark.parametrize("shape", [(1,), (), (1, "N"), ("rows", "N"), ("N",)])
+def test_a_bias_that_broadcasts_is_added(operators, N, K, shape):
+    """With the augmented product (N = 2 K) and with the rank-R term apart: a bias is whatever
+    torch adds to [rows, N]."""
+    packed, absmax, x, a, b, _ = layer(N, K)
+    bias = torch.randn([{"N": N, "rows": x.shape[0]}.get(s, s) for s in shape]).bfloat16()
+    assert close(apply(packed, absmax, x, a, b, bias), reference(packed, x, a, b, bias))
