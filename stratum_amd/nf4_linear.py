@@ -160,8 +160,10 @@ class _NF4LinearFn(torch.autograd.Function):
                     dequantize_4bit(packed, absmax=absmax, blocksize=ctx.blocksize, dtype=dy2.dtype, shape=ctx.shape)
                 ctx.w = None
                 if u is not None:
-                    # rank-R term, then the base GEMM into it
-                    dx = (lora_up(u, lora_a, transposed=True) if lora_supported(u.shape[1], K, u.shape[0])
+                    # rank-R term, then the base GEMM into it; with create_graph torch's product,
+                    # which keeps the graph to A
+                    own = lora_supported(u.shape[1], K, u.shape[0]) and not torch.is_grad_enabled()
+                    dx = (lora_up(u, lora_a, transposed=True) if own
                           else u @ lora_a.to(dy2.dtype)).addmm_(dy2, w)
                 else:
                     dx = dy2 @ w

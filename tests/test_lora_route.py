@@ -97,3 +97,17 @@ def test_a_bias_that_broadcasts_is_added(operators, N, K, shape):
     packed, absmax, x, a, b, _ = layer(N, K)
     bias = torch.randn([{"N": N, "rows": x.shape[0]}.get(s, s) for s in shape]).bfloat16()
     assert close(apply(packed, absmax, x, a, b, bias), reference(packed, x, a, b, bias))
+
+
+@pytest.mark.parametrize("N,K", [(256, 128), (128, 128)])
+def test_input_gradient_stays_differentiable_in_lora_a(operators, N, K):
+    """A gradient penalty: with create_graph, dX = dY W + U A keeps its graph to A."""
+    packed, absmax, x, a, b, dy = layer(N, K)
+    x.requires_grad_(True), a.requires_grad_(True)
+    dx, = torch.autograd.grad(apply(packed, absmax, x, a, b), x, dy, create_graph=True)
+    da, = torch.autograd.grad(dx, a, torch.ones_like(dx))
+    u = 2.0 * dy.float() @ b.float()
+    assert close(da, u.t() @ torch.ones(x.shape))
+    del operators[:]
+    torch.autograd.grad(apply(packed, absmax, x, a, b), (x, a), dy)
+    assert "lora_up" in operators  # a plain backward runs the kernel
