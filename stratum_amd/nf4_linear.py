@@ -42,8 +42,9 @@ import torch.nn.functional as F
 
 import os
 
-from .functional import (QuantState, dequantize_4bit, dequantize_4bit_aug, fused_supported, lora_aug_supported, lora_da,
-                         lora_down, lora_down_aug, lora_dy, lora_supported, lora_up, nf4_gemm_bwd_dx, nf4_gemm_fwd)
+from .functional import (QuantState, _rows, dequantize_4bit, dequantize_4bit_aug, fused_supported, lora_aug_supported,
+                         lora_da, lora_down, lora_down_aug, lora_dy, lora_supported, lora_up, nf4_gemm_bwd_dx,
+                         nf4_gemm_fwd)
 
 _DEFAULT_FUSED_MAX_ROWS = 768
 # With a LoRA adapter the fused kernels fold the rank-R terms into their
@@ -97,7 +98,7 @@ class _NF4LinearFn(torch.autograd.Function):
         t = xa = None
         if lora_a is not None:
             if not fused and _augment(x, packed, absmax, shape, lora_a, lora_b, w_dense):
-                t, xa = lora_down_aug(x if x.dim() == 2 else x.reshape(-1, x.shape[-1]), lora_a, scaling)
+                t, xa = lora_down_aug(_rows(x, x.shape[-1]), lora_a, scaling)
             elif lora_supported(lora_a.shape[0], x.shape[-1], x.numel() // max(x.shape[-1], 1)):
                 t = lora_down(x, lora_a, scaling)
             else:
@@ -140,7 +141,7 @@ class _NF4LinearFn(torch.autograd.Function):
     def backward(ctx, dy):
         x, packed, absmax, lora_a, lora_b, t = ctx.saved_tensors
         N, K = ctx.shape
-        dy2 = (dy if dy.dim() == 2 else dy.reshape(-1, N)).contiguous()
+        dy2 = _rows(dy, N).contiguous()
         u = d_b = None
         if lora_a is not None:
             if lora_supported(lora_a.shape[0], N, dy2.shape[0]):
@@ -172,7 +173,7 @@ class _NF4LinearFn(torch.autograd.Function):
         d_bias = dy2.sum(0).to(dy.dtype) if ctx.has_bias_grad else None
         d_a = None
         if lora_a is not None:
-            x2 = x if x.dim() == 2 else x.reshape(-1, K)
+            x2 = _rows(x, K)
             if ctx.needs_input_grad[6]:
                 d_a = lora_da(u, x2) if lora_supported(lora_a.shape[0], K, x2.shape[0]) else u.t() @ x2  # [R, K]
                 d_a = d_a.to(lora_a.dtype)

@@ -498,3 +498,13 @@ def test_dequantize_host_arguments_and_pageable_memory(L):
     assert L.stm_nf4_dequantize_host(1, ptrs, ptrs, n, 64, ptrs, 0, None) == -2   # pageable
     assert "pinned" in _err(L)
     assert L.stm_event_done(None) == -1
+
+
+def test_a_matrix_without_columns_is_refused():
+    """As a reshape to [-1, 0] refuses it, 2-D or not; no rows are fine."""
+    import torch
+    from stratum_amd.functional import _rows
+    for shape in ((5, 0), (2, 3, 0)):
+        with pytest.raises(RuntimeError):
+            _rows(torch.empty(shape), 0)
+    assert _rows(torch.empty(0, 4), 4).shape == (0, 4) and _rows(torch.empty(2, 0, 4), 4).shape == (0, 4)
