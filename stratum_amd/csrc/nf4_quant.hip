@@ -539,9 +539,11 @@ __global__ __launch_bounds__(256) void k_dequantize_many(DequantMany m) {
 // weight crosses the host link once, as the kernel's own reads, with no device
 // copy of the payload. The link bounds it (54 GB/s measured, the rate of one
 // large copy), so a small persistent grid does: kHostWgs work-groups of four
-// waves keep 1 MB of reads in flight, and the other CUs stay free for kernels of
-// other streams. A layer of seven projections (8.8 MB packed): 165 us, against
-// 315 us as 14 uploads and a batched dequantize.
+// waves keep 1 MB of reads in flight. They hold up to that many CUs for the whole
+// transfer, which a persistent GEMM on another stream has to wait for, so the
+// caller takes this kernel where nothing is meant to run beside it. A layer of
+// seven projections (8.8 MB packed): 165 us, against 315 us as 14 uploads and a
+// batched dequantize.
 template <int DT, int U>
 __global__ __launch_bounds__(256) void k_dequantize_many_host(DequantMany m) {
     __shared__ float2 lut[256];

@@ -314,3 +314,16 @@ def test_nf4_linear_shape_metadata_without_gpu():
     st = QuantState(absmax=torch.ones(4), shape=(16, 32), blocksize=64, quant_type="nf4", dtype=torch.float16)
     lin = NF4Linear(torch.zeros(256, 1, dtype=torch.uint8), st, bias=torch.zeros(16, dtype=torch.float16))
     assert lin.in_features == 32 and lin.out_features == 16 and not lin.bias.requires_grad
+
+
+@pytest.mark.parametrize("readers,host", [([], True), (["another stream"], False)])
+def test_pinned_payloads_are_read_in_place_only_for_the_staging_stream_itself(monkeypatch, readers, host):
+    """For a reader on another stream the payload is copied, so that its transfer takes no compute
+    units from what that stream runs meanwhile; a prefetched payload is never read in place."""
+    seen = []
+    monkeypatch.setattr(U, "_materialise_group", lambda members, device, consumers, on_host: seen.append((len(members), on_host)))
+    monkeypatch.setattr(torch.cuda, "device", lambda device: mock.MagicMock())
+    fresh = [(None, None, nf4_payload(), None)] * 3
+    fetched = [(None, None, nf4_payload(), ("codes", "absmax"))] * 2
+    assert U._materialise_nf4(fresh + fetched, torch.device("cuda", 0), readers) == 5
+    assert sorted(seen) == ([(2, False), (3, True)] if host else [(5, False)])
