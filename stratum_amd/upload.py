@@ -40,9 +40,10 @@ from __future__ import annotations
 
 import hashlib
 import re
-import threading
+import sys
 import time
 import weakref
+from collections import deque
 from dataclasses import dataclass
 from pathlib import Path
 from typing import Iterable, Iterator, Optional, Sequence
@@ -475,10 +476,13 @@ def _upload_nf4(payload: NF4Payload, device: torch.device):
     return (payload.quantized.to(device, non_blocking=True), payload.absmax.to(device, non_blocking=True))
 
 
-# Payloads that a launch still reads from pinned memory, with the event behind
-# it: a payload that its owner drops meanwhile must not be reused by the host.
-_host_reads: list = []
-_host_reads_lock = threading.Lock()
+# What launches still read from pinned memory: the event behind each launch, the
+# tensors, and weak references to their payloads. A payload that its owner drops
+# meanwhile keeps its memory until the launch has run, and no longer than its
+# owner where it has: the next staging call lets go of the tensors, and so does
+# the end of any of these payloads. A callback can run at any point of any
+# thread, so there is no lock: deque's own operations are atomic.
+_host_reads: deque = deque()
 
 
 def _keep_while_read(payloads: list, device: torch.device) -> None:
@@ -486,15 +490,21 @@ def _keep_while_read(payloads: list, device: torch.device) -> None:
         return  # what a graph reads is its owner's to keep, as with a captured copy
     done = torch.cuda.Event()
     done.record(torch.cuda.current_stream(device))
-    with _host_reads_lock:
-        _host_reads.append((done, payloads))
+    _host_reads.append((done, [(p.quantized, p.absmax) for p in payloads],
+                        [weakref.ref(p, _release_host_reads) for p in payloads]))
 
 
-def _release_host_reads() -> None:
-    if not _host_reads:
+def _release_host_reads(_payload=None) -> None:
+    """Let go of what the launches that have run did read."""
+    if sys.is_finalizing():
         return
-    with _host_reads_lock:
-        _host_reads[:] = [r for r in _host_reads if _lib.lib().stm_event_done(r[0].cuda_event) == 0]
+    for _ in range(len(_host_reads)):
+        try:
+            read = _host_reads.popleft()
+        except IndexError:
+            return  # another thread took the last
+        if _lib.lib().stm_event_done(read[0].cuda_event) == 0:
+            _host_reads.append(read)
 
 
 def _materialise_nf4(entries: list, device: torch.device, consumers: list) -> int:
@@ -531,10 +541,10 @@ def _materialise_group(members: list, device: torch.device, consumers: list, on_
 
     weights = None
     if on_host:
-        sources = [(payload.quantized, payload.absmax) for _, _, payload, _ in members]
-        weights = dequantize_4bit_host(items(sources), device)
+        weights = dequantize_4bit_host(items([(payload.quantized, payload.absmax) for _, _, payload, _ in members]),
+                                       device)
         if weights is not None:
-            _keep_while_read(sources, device)
+            _keep_while_read([payload for _, _, payload, _ in members], device)
     if weights is None:
         weights = dequantize_4bit_many(items([prefetched if prefetched is not None else _upload_nf4(payload, device)
                                               for _, _, payload, prefetched in members]))
@@ -635,6 +645,7 @@ def upload_stream(module: torch.nn.Module, device_id: int, *, verbose: bool = Tr
     device = _cuda(device_id)
     placed = ensure_weights(module, device_id)
     torch.cuda.current_stream(device).synchronize()
+    _release_host_reads()
     seconds = time.time() - t0
     log_event("upload_stream", device=device_id, tensors=placed, seconds=round(seconds, 1))
     if verbose:

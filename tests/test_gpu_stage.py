@@ -274,3 +274,22 @@ def test_ensure_weights_inside_a_captured_graph_reads_the_payload_on_each_replay
         graph.replay()
         torch.cuda.synchronize()
         assert all(torch.equal(h, w) for h, w in zip(held, want) if h.dim() == 2)
+
+
+@pytest.mark.parametrize("way", ["upload_stream", "ensure_weights"])
+def test_payloads_leave_pinned_memory_with_their_module(cuda, way):
+    import gc
+    import weakref
+    import stratum_amd.upload as U
+    layer = _two_layers()[0]
+    payloads = [getattr(p, U.NF4_ATTR) for p in layer.parameters() if hasattr(p, U.NF4_ATTR)]
+    held = [weakref.ref(t) for payload in payloads for t in (payload.quantized, payload.absmax)]
+    if way == "upload_stream":
+        U.upload_stream(layer, 0, verbose=False)
+    else:
+        U.ensure_weights(layer, 0)
+        torch.cuda.synchronize()
+    assert held and all(r() is not None and r().is_pinned() for r in held)
+    del layer, payloads
+    gc.collect()
+    assert all(r() is None for r in held)

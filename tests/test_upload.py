@@ -5,6 +5,8 @@ free_weights scope, empty prefetch, prefetch + ensure chaining, cache v1
 accept/reject, FP16-staged lifecycle, 2-D / 3-D prepare with the quantizer
 replaced by a recording stand-in, and buffer snapshot/restore."""
 
+import gc
+import weakref
 from pathlib import Path
 from unittest import mock
 
@@ -327,3 +329,48 @@ def test_pinned_payloads_are_read_in_place_only_for_the_staging_stream_itself(mo
     fetched = [(None, None, nf4_payload(), ("codes", "absmax"))] * 2
     assert U._materialise_nf4(fresh + fetched, torch.device("cuda", 0), readers) == 5
     assert sorted(seen) == ([(2, False), (3, True)] if host else [(5, False)])
+
+
+class _FakeReads:
+    """Events that are done when the test says so, in place of the GPU's."""
+
+    def __init__(self, monkeypatch):
+        self.done = False
+        reads = self
+
+        class Event:
+            cuda_event = 1
+
+            def record(self, stream):
+                pass
+
+        class Lib:
+            def stm_event_done(self, event):
+                return int(reads.done)
+
+        monkeypatch.setattr(torch.cuda, "Event", Event)
+        monkeypatch.setattr(torch.cuda, "current_stream", lambda device=None: None)
+        monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+        monkeypatch.setattr(U._lib, "lib", lambda: Lib())
+
+
+def test_a_payload_that_a_launch_has_read_goes_with_its_owner(monkeypatch):
+    """Nothing but its owner holds a payload once the launch has run: dropping the owner frees
+    it, with no staging call after it; before that the launch's hold keeps its memory."""
+    gpu = _FakeReads(monkeypatch)
+    monkeypatch.setattr(U, "dequantize_4bit_host", lambda items, device: [torch.empty(2, 2) for _ in items])
+    for done in (True, False):
+        layer = nn.Module()
+        layer.weight = nn.Parameter(torch.empty(0, dtype=torch.float16), requires_grad=False)
+        setattr(layer.weight, NF4_ATTR, nf4_payload())
+        slot = mock.Mock(owner=layer)
+        slot.name = "weight"
+        U._materialise_group([(slot, layer.weight, getattr(layer.weight, NF4_ATTR), None)], torch.device("cpu"), [], True)
+        held = weakref.ref(getattr(layer.weight, NF4_ATTR).quantized)
+        gpu.done = done
+        del layer, slot
+        gc.collect()
+        assert (held() is None) == done
+    gpu.done = True
+    U.free_weights(nn.Module())  # the next staging call lets go of what was still being read
+    assert held() is None
