@@ -3347,10 +3347,14 @@ int launch_gemv_ks(const GemmArgs& g, int cfg, int dtype, hipStream_t stream, in
 // (0: unknown) of at most M rows each, or 0 where one work-group per CU over
 // whole-reduction items (k_gemv_fwd) is estimated faster, in the same unit:
 // two tile-groups per group, the fixed cost once. Few experts leave that
-// kernel's 256-row items on few CUs ([1536, 2048] over 8 of 128 experts: 17.7
-// against 8.0 us); many pay the split-free kernel's fixed cost once per
-// work-group, for which its estimate counts 1.3 times (30 experts: 20.5
-// against 23.0 us).
+// kernel's 256-row items on few CUs; many pay the split-free kernel's fixed cost
+// once per work-group, for which its estimate counts 1.4 times: both timed over
+// 446 calls (banks [2 I, H] and [H, I] of 32-128 experts, H 1024 and 2048,
+// I 384-1024, 2-128 experts with 1-16 rows), the estimates without the factor
+// stand 1.43 or more apart where this kernel is faster (us: [1536, 2048] over
+// 8 experts 7.6 against 16.8, [2048, 768] over 16 6.6 / 8.9, [1024, 1024] over
+// 31 7.5 / 10.4) and 1.32 or less where it is not ([1536, 2048] over 29 20.9 /
+// 18.4, over 53 35.8 / 33.4), with one exception of 4 % ([2048, 2048] over 45).
 int gemv_ks_grouped_config(int64_t M, int hits, int64_t N, int64_t K) {
     if (!STM_GEMV_KS || M < 1 || M > 16 || hits < 1) return 0;
     const int64_t cus = device_cus(), items = hits * ((N + GvCfg<1, 256>::ROWS - 1) / GvCfg<1, 256>::ROWS);
@@ -3359,7 +3363,7 @@ int gemv_ks_grouped_config(int64_t M, int hits, int64_t N, int64_t K) {
     for (const auto& c : kKsConfigs) {
         int64_t blocks;
         const double t = gemv_ks_time(c, hits, N, K, cus, &blocks);
-        if (M <= c[2] && 1.3 * t < best_t) best_t = 1.3 * t, best = c[0] | c[1] << 4 | c[2] << 8;
+        if (M <= c[2] && 1.4 * t < best_t) best_t = 1.4 * t, best = c[0] | c[1] << 4 | c[2] << 8;
     }
     return best;
 }

@@ -296,6 +296,25 @@ def test_grouped_forward_small_rows_per_expert(cuda, monkeypatch, dtype, counts,
     assert rel(y, yt) <= TOL[dtype] / 4
 
 
+@pytest.mark.parametrize("experts,N,K,kernel", [
+    (8, 1536, 2048, "k_gemv_ks"), (29, 1536, 2048, "k_gemv_fwd"), (53, 1536, 2048, "k_gemv_fwd"),
+    (16, 2048, 768, "k_gemv_ks"), (31, 1024, 1024, "k_gemv_ks"),
+])
+def test_grouped_small_rows_take_the_faster_kernel(cuda, experts, N, K, kernel):
+    """The split-free kernel for few experts with rows, the walking one for many, as timed."""
+    from stratum_amd.functional import nf4_grouped_gemm
+    packed = torch.randint(0, 256, (experts * N * K // 2, 1), dtype=torch.uint8, device=cuda)
+    absmax = torch.rand(experts * N * K // 64, device=cuda)
+    x = seeded((2 * experts, K), 85, 1.0, torch.bfloat16).to(cuda)
+    offsets = torch.arange(0, 2 * experts + 1, 2, dtype=torch.int32)
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as prof:
+        nf4_grouped_gemm(x, packed, absmax, offsets, (N, K))
+        torch.cuda.synchronize()
+    names = [e.name for e in prof.events() if "k_gemv" in e.name]
+    if names:  # the profiler saw device kernels
+        assert len(names) == 1 and kernel in names[0], names
+
+
 @pytest.mark.parametrize("host_counts", [[0, 4, 0, 0, 0, 0], [4, 4, 4, 4, 4, 4], None])
 def test_grouped_small_rows_follow_the_device_offsets(cuda, host_counts):
     """The host's copy of the offsets sizes the launch (here: fewer or more experts
