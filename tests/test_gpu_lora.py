@@ -225,3 +225,32 @@ def test_library_path_step_with_and_without_augmentation(cuda, dtype, keep, N, K
     ref.backward(dy.float().reshape(-1, N))
     for got, want in ((y, ref), (x.grad, xf.grad), (lin.lora_A.grad, a.grad), (lin.lora_B.grad, b.grad)):
         assert rel(got.detach().reshape(want.shape), want.detach()) <= TOL[dtype]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("N,K,M,R", [(768, 384, 123, 32), (640, 320, 1100, 32), (704, 320, 65, 16), (2048, 1024, 1500, 16)])
+def test_augmented_forward_is_one_rounding_of_one_sum(cuda, dtype, N, K, M, R, monkeypatch):
+    """Y of the product over [x | t] and [W | B]: an fp32 sum of K + R products, rounded once. Each
+    value is within one unit in the last place of the exact one plus 2^-23 (K + 64) of the sum of
+    magnitudes (an addition is off by at most 2^-23 of it, whatever the order and the rounding)."""
+    import importlib
+    from stratum_amd.functional import dequantize_4bit, lora_down, quantize_4bit
+    from stratum_amd.nf4_linear import NF4LoRALinear
+    module, taken = importlib.import_module("stratum_amd.nf4_linear"), []
+    real = module._augment
+    monkeypatch.setattr(module, "_augment", lambda *args: taken.append(real(*args)) or taken[-1])
+    monkeypatch.setenv("STRATUM_NF4_FUSED_MAX_ROWS", "0")
+    q, st = quantize_4bit(seeded((N, K), 21, 0.02, torch.float16, cuda))
+    lin = NF4LoRALinear(q, st, r=R, lora_alpha=float(R), dtype=dtype)
+    with torch.no_grad():
+        lin.lora_A.copy_(seeded((R, K), 22, 0.05, dtype, cuda))
+        lin.lora_B.copy_(seeded((N, R), 23, 0.05, dtype, cuda))
+        x = seeded((M, K), 24, 1.0, dtype, cuda)
+        y = lin(x)
+        assert torch.equal(y, lin(x)) and taken == [True, True]
+        t = lora_down(x, lin.lora_A).double()
+        w, b = (v.double().t().contiguous() for v in (dequantize_4bit(q, st, dtype=dtype), lin.lora_B))
+        exact, scale = x.double() @ w + t @ b, x.double().abs() @ w.abs() + t.abs() @ b.abs()
+    unit = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
+    tiny = 0.0 if dtype == torch.bfloat16 else 2.0 ** -25  # half the spacing of fp16's subnormals
+    assert bool(((y.double() - exact).abs() <= unit * exact.abs() + (K + 64) * 2.0 ** -23 * scale + tiny).all())

@@ -293,3 +293,51 @@ def test_payloads_leave_pinned_memory_with_their_module(cuda, way):
     del layer, payloads
     gc.collect()
     assert all(r() is None for r in held)
+
+
+def _stage_of(shapes, seed):
+    import stratum_amd.upload as U
+    m = nn.Module()
+    for j, shape in enumerate(shapes):
+        m.register_parameter("w%d" % j, nn.Parameter(seeded(shape, seed + j, 0.02, torch.float16), requires_grad=False))
+    want = [oracle_bits(p) for p in m.parameters()]
+    U.prepare_nf4(m, verbose=False, min_numel=1)
+    return m, want
+
+
+@pytest.mark.parametrize("way,shapes,in_place,copied", [
+    ("plain", [(64, 128), (32, 64)], 1, 0),
+    ("side stream", [(64, 128), (32, 64)], 0, 1),
+    ("pageable", [(64, 128), (32, 64)], 0, 1),
+    ("plain", [(64, 128), (63, 65)], 0, 1),            # 4095 elements: not whole groups of 8
+    ("plain", [(16, 64)] * 33, 2, 0),                  # 32 tensors a launch, and one more
+    ("side stream", [(16, 64)] * 33, 0, 2),
+    ("pageable", [(16, 64)] * 33, 1, 1),               # the pageable one is among the first 32
+])
+def test_every_way_to_materialise_payloads(cuda, monkeypatch, way, shapes, in_place, copied):
+    """Launches that read pinned memory and launches on device copies, by way, each bit-exact."""
+    import stratum_amd.upload as U
+    m, want = _stage_of(shapes, 40)
+    if way == "pageable":
+        payload = getattr(m.w1, U.NF4_ATTR)
+        payload.quantized = payload.quantized.clone()
+        assert not payload.quantized.is_pinned()
+    ran = []
+    for name in ("dequantize_4bit_host", "dequantize_4bit_many"):
+        def call(*args, _real=getattr(U, name), _name=name):
+            out = _real(*args)
+            if out is not None:
+                ran.append(_name)
+            return out
+        monkeypatch.setattr(U, name, call)
+    stream = torch.cuda.Stream() if way == "side stream" else torch.cuda.current_stream()
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as prof:
+        with torch.cuda.stream(stream):
+            assert U.ensure_weights(m, 0) == len(shapes)
+        torch.cuda.synchronize()
+    assert ran.count("dequantize_4bit_host") == in_place and ran.count("dequantize_4bit_many") == copied
+    names = [e.name for e in prof.events() if "k_dequantize" in e.name]
+    if names and copied and all(a * b % 64 == 0 for a, b in shapes):  # the profiler saw device kernels
+        assert sum("k_dequantize_many_host" not in n and "k_dequantize_many" in n for n in names) == copied, names
+    for p, w in zip(m.parameters(), want):
+        assert torch.equal(p.data.cpu().view(torch.int16), w)
