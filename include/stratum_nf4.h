@@ -97,8 +97,10 @@ int stm_nf4_dequantize_many(int count, const uint8_t* const* packed, const float
  * absmax[t] are host addresses (hipHostMalloc) that the kernel reads over the
  * host link, so the payload crosses it once and needs no device copy
  * (the two uploads and the dequantize per parameter of stratum/upload.py
- * ensure_weights, :1022-1044). Same results, bit for bit. The caller keeps the
- * memory allocated until the launch has run. STM_ERR_UNSUPPORTED, before any
+ * ensure_weights, :1022-1044). Same results, bit for bit. The launch holds up to
+ * 128 compute units for the whole transfer, so it suits a stage that nothing is
+ * meant to run beside. The caller keeps the memory allocated until the launch has
+ * run. STM_ERR_UNSUPPORTED, before any
  * launch, for more than 32 tensors, n[t] % 8 != 0, unaligned pointers (4 bytes
  * in, 16 out) and memory that is not one pinned host range.
  */

@@ -78,7 +78,7 @@ struct LoraArgs {
 };
 
 // RP = R rounded up to 16 (zero ranks padded). ROW / COL select the products; COPY also
-// writes Z into zcopy as it passes (X [8192, 4096]: 26 us, 15 without; a copy of its own
+// writes Z into zcopy as it passes (X [8192, 4096]: 25 us, 15 without; a copy of its own
 // would read X again).
 template <typename Tr, int RP, bool ROW, bool COL, bool COPY = false>
 __global__ __launch_bounds__(256, 2) void k_lora_pass(LoraArgs g) {
@@ -474,8 +474,9 @@ void launch_down_rows(const void* X, const void* A, void* T, int64_t M, int64_t 
 // MFMA row i of fragment f is column 32 (f / 2) + 8 (i / 4) + 4 (f % 2) + i % 4, so lane
 // (lr, lh) ends with two 16-byte chunks of row lr: lh and lh + 4 of the row's 128 bytes.
 // Lanes 8 apart trade one chunk each, and every store instruction then writes 8 whole
-// 128-byte lines. W [14336, 4096] at 8192 rows (235 MB): 40 us (5.9 TB/s)
-// against 72 for a plain library product; LT, [8192, 4096]: 16.7 against 25.7.
+// 128-byte lines. In a traced LoRA step, Y [8192, 14336] (235 MB): 61 us (3.9 TB/s)
+// against 85 for a plain library product; LT, [8192, 4096]: 18.2 against 32.7. Repeated
+// by itself the first takes 40 us (5.9 TB/s), the product 72.
 template <typename Tr, bool LT>
 __global__ __launch_bounds__(256) void k_lora_up(const uint16_t* __restrict__ T, const uint16_t* __restrict__ L,
                                                  const uint16_t* __restrict__ bias, uint16_t* __restrict__ Y,

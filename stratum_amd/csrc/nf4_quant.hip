@@ -573,7 +573,7 @@ __global__ __launch_bounds__(256) void k_dequantize_generic(const uint8_t* __res
 // k_dequantize into rows of cols + 64 columns: after the weight's cols (a multiple of 64)
 // come the rank columns of L [rows, R] and zeros, so one product over cols + 64 columns
 // adds the LoRA term. Word g of the flat list is piece g % (wpr + 8) of row g / (wpr + 8).
-// Bound by the write: [14336, 4096] in 31 us (153 MB moved, 4.9 TB/s; k_dequantize 26).
+// Bound by the write: [14336, 4096] in 32 us (153 MB moved, 4.8 TB/s; k_dequantize 26).
 template <int DT, int U>
 __global__ __launch_bounds__(256) void k_dequantize_aug(const uint32_t* __restrict__ q,
                                                         const float* __restrict__ absmax,

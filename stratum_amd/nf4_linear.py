@@ -9,8 +9,9 @@ paths for its row count M (tokens), measured on MI355X:
 * M <= ``fused_max_rows()`` (default 768; 1024 with a LoRA adapter): one
   fused dequant-GEMM forward and one fused dequant-GEMM for ``dX = dY . W``;
   the dequantized weight never exists in HBM, and the packed weight (0.56 B/element) is all the weight
-  traffic -- forward plus input gradient, the fused kernels are faster there
-  (at M = 768 on the 8B-class weights: 0.22 against 0.25 ms);
+  traffic -- forward plus input gradient, calls in sequence, take no longer there than on the other path
+  (at M = 768 0.22 ms by either on the 8B-class weights; the forward alone can: 62 us against 42 on
+  [4096, 4096] at M = 768);
 * larger M: ``dequantize_4bit`` into a temporary, then the library GEMM
   (hipBLASLt), whose forward is 1.2-1.3x faster than the fused kernel at
   M = 2048..8192, because the dequantization is paid once for all rows instead
@@ -48,10 +49,12 @@ from .functional import (QuantState, _rows, dequantize_4bit, dequantize_4bit_aug
 
 _DEFAULT_FUSED_MAX_ROWS = 768
 # With a LoRA adapter the fused kernels fold the rank-R terms into their
-# epilogues, while the library path pays extra passes over Y and dX for them, so
-# the crossover sits higher: forward + backward on the 8B-class weights at
-# M = 1024, 0.30-0.32 ms fused against 0.33 ms; even at 1536-2048 rows;
-# library ahead from 4096 rows (8192: 1.81 against 1.70 ms).
+# epilogues, and the library path's step has more launches: 40 us more of the
+# host's time. Forward + backward, calls in sequence, us, fused / library:
+# at 768 rows [1024, 1024] 206 / 252, [4096, 4096] 211 / 249, [4096, 14336]
+# 261 / 264, [14336, 4096] 262 / 261; at 1024 rows 201 / 250, 200 / 251,
+# 299 / 294, 324 / 288. (GPU time alone has the library ahead from about 384
+# rows on most weights: [4096, 4096] at 768 163 / 112.)
 _DEFAULT_FUSED_MAX_ROWS_LORA = 1024
 
 
@@ -76,10 +79,12 @@ def _augment(x, packed, absmax, shape, lora_a, lora_b, w_dense) -> bool:
     """Whether the library path's forward runs one product over K + 64 columns, [x | t] [W | B]^T.
 
     It saves the rank-R term's write of Y and the base product's read of it (4 N bytes a row) for a
-    copy of x (2 K bytes a row) and 64 / K more products, so it is taken for N >= 2 K.
-    W [14336, 4096] at 8192 rows, us: product 656 -> 616, no 40 for the term, copy 15 -> 26,
-    dequantize 26 -> 31. At N = K the library product over K + 64 columns takes back what is
-    saved ([4096, 4096] at 4096 rows: 92 + 11 for product and term, 88 + 12 with the copy)."""
+    copy of x (2 K bytes a row) and 64 / K more products, so it is taken for N >= 2 K. One traced step,
+    W [14336, 4096] at 8192 rows, us: product 702 -> 659, no 61 for the term, the pass over x 15 -> 25,
+    dequantize 26 -> 32. GPU time of the whole step against the term apart, 1025-8192 rows, K 512-4096:
+    N > 2 K 0.73-1.04, N = 2 K 0.91-1.05, N = 1.5 K 0.92-1.00, N = K 0.95-1.07; over 1 where the library
+    has a slower product for K + 64 columns ([2048, 1024] and [3072, 1024] at 5800 rows, [1024, 1024] at
+    4096), which no rule on sizes foretells."""
     N, K = shape
     rows = x.numel() // max(K, 1)
     return (N >= 2 * K and rows > 64 and w_dense is None and packed.dtype == torch.uint8
